@@ -207,6 +207,7 @@ constexpr int kTsHistThreads = 256;
 constexpr int kTsLoads = 4;  // particles per thread per histogram iteration
 constexpr int kTsAhead = 8;  // rounds of 64 particles in flight per scatter wave
 constexpr int kTsMatch = 4;  // tiles matched one by one per scatter round
+constexpr int kTsHistMatch = 8;  // the same per histogram wave
 
 // rounds of 64 particles per chunk: at least 16, more when the chunk x tile
 // count table would exceed 2^24 entries
@@ -262,15 +263,20 @@ ts_hist_kernel(const float* __restrict__ x, const float* __restrict__ y, int n, 
         for (int k = 0; k < kTsLoads; ++k) {
             const bool valid = i0 + k * kTsHistThreads + (int)threadIdx.x < end;
             const int t = valid ? tile_id(px[k], py[k], tm) : -1;
-            // one LDS atomic per distinct tile of the wave
+            // A nearly sorted wave spans few tiles: one LDS atomic for each of
+            // its first kTsHistMatch distinct tiles.  Lanes still pending add for
+            // themselves: in a mixed wave they name many tiles, so the adds
+            // rarely meet, while matching them one by one took up to 64 rounds
+            // (3.1 M particles in no order over 192 tiles: 86 -> 16 us).
             unsigned long long todo = __ballot(valid);
-            while (todo) {
+            for (int it = 0; it < kTsHistMatch && todo; ++it) {
                 const int leader = __ffsll((long long)todo) - 1;
                 const int lt = __builtin_amdgcn_readlane(t, leader);
                 const unsigned long long mk = __ballot(t == lt) & todo;
                 if (lane == leader) atomicAdd(&h[lt], (uint32_t)__popcll(mk));
                 todo &= ~mk;
             }
+            if ((todo >> lane) & 1ull) atomicAdd(&h[t], 1u);
         }
     }
     __syncthreads();
@@ -282,11 +288,20 @@ ts_hist_kernel(const float* __restrict__ x, const float* __restrict__ y, int n, 
 // Offsets of the chunk-major count table T[chunk][tile] in tile-major order:
 // off(t, c) = base(t) + sum_{c' < c} T[c'][t], base(t) = sum_{t' < t} total(t').
 // Chunks are taken kTsColBlock at a time: ts_colsum sums each (block, tile)
-// column segment, ts_colscan scans the block sums per tile (and yields the
-// tile totals), the totals are scanned into base(t), and ts_colapply rewrites
-// T in place with the offsets.  Every pass reads rows of T, coalesced across
-// the tiles.
+// column segment, the block sums become each segment's first offset, and
+// ts_colapply rewrites T in place.  Every pass reads rows of T, coalesced
+// across the tiles, kTsColLoads rows in flight per thread.  The middle pass is
+// one workgroup (ts_scan) while its counters are few, else a scan per tile
+// (ts_colscan) and a device-wide scan of the tile totals: for small sorts the
+// launches are the cost.
 constexpr int kTsColBlock = 64;
+constexpr int kTsColLoads = 16;
+constexpr int kTsScanThreads = 1024;
+// counters that one workgroup scans (16 M particles on 256 tiles are 64 k of
+// them, 64 rows a thread): 4.4 us at 3 M particles and 192 tiles, where the
+// per-tile scan, the three launches of the device-wide one and the offsets'
+// copy it replaces took 31 us
+constexpr int64_t kTsScanMax = 1 << 16;
 
 __global__ void ts_colsum_kernel(const uint32_t* __restrict__ table, int nchunks, int ntiles,
                                  uint32_t* __restrict__ bsum) {
@@ -294,8 +309,80 @@ __global__ void ts_colsum_kernel(const uint32_t* __restrict__ table, int nchunks
     if (t >= ntiles) return;
     const int c0 = blockIdx.y * kTsColBlock, c1 = min(nchunks, c0 + kTsColBlock);
     uint32_t v = 0;
-    for (int c = c0; c < c1; ++c) v += table[(size_t)c * ntiles + t];
+    for (int c = c0; c < c1; c += kTsColLoads) {
+        uint32_t e[kTsColLoads];
+#pragma unroll
+        for (int k = 0; k < kTsColLoads; ++k)
+            e[k] = c + k < c1 ? table[(size_t)(c + k) * ntiles + t] : 0u;
+#pragma unroll
+        for (int k = 0; k < kTsColLoads; ++k) v += e[k];
+    }
     bsum[(size_t)blockIdx.y * ntiles + t] = v;
+}
+
+// rows [r0, r1) of column t of a[row][ntiles] become the running offsets from
+// `run` on; returns the offset past the last
+__device__ __forceinline__ uint32_t ts_prefix_column(uint32_t* __restrict__ a, int r0, int r1,
+                                                     int ntiles, int t, uint32_t run) {
+    for (int r = r0; r < r1; r += kTsColLoads) {
+        uint32_t e[kTsColLoads];
+#pragma unroll
+        for (int k = 0; k < kTsColLoads; ++k)
+            e[k] = r + k < r1 ? a[(size_t)(r + k) * ntiles + t] : 0u;
+#pragma unroll
+        for (int k = 0; k < kTsColLoads; ++k) {
+            if (r + k < r1) a[(size_t)(r + k) * ntiles + t] = run;
+            run += e[k];
+        }
+    }
+    return run;
+}
+
+// ntiles <= kTsScanThreads: bsum[b][t] -> base(t) + the sum over the blocks
+// before b, and off.  The workgroup splits the blocks over G groups of ntiles
+// threads, scans the groups' sums per tile, then the tile totals.
+__global__ void __launch_bounds__(kTsScanThreads)
+ts_scan_kernel(uint32_t* __restrict__ bsum, int nblocks, int ntiles, int n,
+               int32_t* __restrict__ off) {
+    __shared__ uint32_t part[kTsScanThreads];  // [group][tile]
+    __shared__ uint32_t base[kTsScanThreads];
+    __shared__ uint32_t wsum[kTsScanThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int G = kTsScanThreads / ntiles, grp = tid / ntiles, t = tid - grp * ntiles;
+    const int per = (nblocks + G - 1) / G;
+    const int b0 = min(grp * per, nblocks), b1 = grp < G ? min(b0 + per, nblocks) : b0;
+    uint32_t v = 0;
+    for (int b = b0; b < b1; b += kTsColLoads) {
+        uint32_t e[kTsColLoads];
+#pragma unroll
+        for (int k = 0; k < kTsColLoads; ++k)
+            e[k] = b + k < b1 ? bsum[(size_t)(b + k) * ntiles + t] : 0u;
+#pragma unroll
+        for (int k = 0; k < kTsColLoads; ++k) v += e[k];
+    }
+    part[tid] = v;
+    __syncthreads();
+    uint32_t total = 0;
+    if (tid < ntiles)
+        for (int g = 0; g < G; ++g) {
+            const uint32_t e = part[g * ntiles + tid];
+            part[g * ntiles + tid] = total;
+            total += e;
+        }
+    uint32_t incl = total;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += o;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    uint32_t before = 0;
+    for (int w = 0; w < wave; ++w) before += wsum[w];
+    base[tid] = before + incl - total;
+    if (tid < ntiles) off[tid] = (int32_t)base[tid];
+    if (tid == 0) off[ntiles] = n;
+    __syncthreads();
+    if (b0 < b1) (void)ts_prefix_column(bsum, b0, b1, ntiles, t, base[t] + part[tid]);
 }
 
 // bsum[b][t] -> exclusive prefix over b; total[t] = column total
@@ -303,28 +390,27 @@ __global__ void ts_colscan_kernel(uint32_t* __restrict__ bsum, int nblocks, int 
                                   uint32_t* __restrict__ total) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ntiles) return;
-    uint32_t run = 0;
-    for (int b = 0; b < nblocks; ++b) {
-        const uint32_t v = bsum[(size_t)b * ntiles + t];
-        bsum[(size_t)b * ntiles + t] = run;
-        run += v;
-    }
-    total[t] = run;
+    total[t] = ts_prefix_column(bsum, 0, nblocks, ntiles, t, 0u);
 }
 
+// base (may be NULL: bsum holds it already) and off: see ts_scan_kernel; the
+// workgroups of the first block also write off
 __global__ void ts_colapply_kernel(uint32_t* __restrict__ table, int nchunks, int ntiles,
                                    const uint32_t* __restrict__ bpre,
-                                   const uint32_t* __restrict__ base) {
+                                   const uint32_t* __restrict__ base, int n,
+                                   int32_t* __restrict__ off) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ntiles) return;
     const int c0 = blockIdx.y * kTsColBlock, c1 = min(nchunks, c0 + kTsColBlock);
-    uint32_t run = base[t] + bpre[(size_t)blockIdx.y * ntiles + t];
-    for (int c = c0; c < c1; ++c) {
-        uint32_t* e = table + (size_t)c * ntiles + t;
-        const uint32_t v = *e;
-        *e = run;
-        run += v;
+    uint32_t run = bpre[(size_t)blockIdx.y * ntiles + t];
+    if (base) {
+        run += base[t];
+        if (blockIdx.y == 0) {
+            off[t] = (int32_t)base[t];
+            if (t == 0) off[ntiles] = n;
+        }
     }
+    (void)ts_prefix_column(table, c0, c1, ntiles, t, run);
 }
 
 struct TsMove {
@@ -420,13 +506,6 @@ ts_scatter_kernel(TsMove m, int n, TileMap tm, int ntiles, int rounds, int tbits
             }
         }
     }
-}
-
-__global__ void ts_offsets_kernel(const uint32_t* __restrict__ base, int ntiles, int n,
-                                  int32_t* __restrict__ off) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < ntiles) off[t] = (int32_t)base[t];
-    if (t == ntiles) off[t] = n;
 }
 
 // ---- SoA permutation ---------------------------------------------------------------
@@ -662,15 +741,18 @@ bool tile_sort_onepass(aw_ctx& c, const aw_particles& src, const aw_particles& d
     const dim3 cg(blocks_for((int64_t)c.ntiles), nblk);
     ts_colsum_kernel<<<cg, kThreads, 0, s>>>(c.sort.table.get(), nchunks, c.ntiles, bsum);
     AW_LAUNCH_CHECK();
-    ts_colscan_kernel<<<blocks_for((int64_t)c.ntiles), kThreads, 0, s>>>(bsum, nblk, c.ntiles,
-                                                                         tbase);
-    AW_LAUNCH_CHECK();
-    exclusive_scan(c, tbase, (int64_t)c.ntiles, s);
+    if (c.ntiles <= kTsScanThreads && (int64_t)nblk * c.ntiles <= kTsScanMax) {
+        ts_scan_kernel<<<1, kTsScanThreads, 0, s>>>(bsum, nblk, c.ntiles, n, off);
+        AW_LAUNCH_CHECK();
+        tbase = nullptr;
+    } else {
+        ts_colscan_kernel<<<blocks_for((int64_t)c.ntiles), kThreads, 0, s>>>(bsum, nblk, c.ntiles,
+                                                                             tbase);
+        AW_LAUNCH_CHECK();
+        exclusive_scan(c, tbase, (int64_t)c.ntiles, s);
+    }
     ts_colapply_kernel<<<cg, kThreads, 0, s>>>(c.sort.table.get(), nchunks, c.ntiles, bsum,
-                                               tbase);
-    AW_LAUNCH_CHECK();
-    ts_offsets_kernel<<<blocks_for((int64_t)c.ntiles + 1), kThreads, 0, s>>>(tbase, c.ntiles, n,
-                                                                           off);
+                                               tbase, n, off);
     AW_LAUNCH_CHECK();
     TsMove m{src.x, src.y, src.ux, src.uy, src.uz, src.w,
              dst.x, dst.y, dst.ux, dst.uy, dst.uz, dst.w, perm};
