@@ -185,7 +185,7 @@ struct EmBatch {
 // scratch of the standalone Darwin operators (aw_deposit_rho_j_amu, ...)
 struct EmScratch {
     DevBuf<unsigned long long> acc;  // up to 8 fixed-point grids
-    DevBuf<unsigned int> bound;      // max|w|, max|u| (float bits)
+    DevBuf<float> bound;             // per-workgroup max|w|, max|u|
     DevBuf<float> cq, cdcu, fpart;   // moment / dcu coefficients, field maxima
     DevBuf<double> inv, dv;          // inverse scales (11), dcu bound inputs (2)
 };
@@ -222,6 +222,7 @@ struct aw_ctx {
     aw::DevBuf<unsigned char> fft_work;
     // workspace
     aw::DevBuf<float> ktmp;                  // complex scratch, 2 floats per mode
+    aw::DevBuf<float> fpack;                 // fields packed per cell for unsorted gathers
     aw::DevBuf<float> rin;                   // R2C input copy (rocFFT may clobber it)
     aw::DevBuf<unsigned long long> acc;      // fixed-point grid accumulator
     aw::DevBuf<double> red;                  // reduction partials
