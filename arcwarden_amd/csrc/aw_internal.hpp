@@ -398,16 +398,16 @@ __device__ __forceinline__ bool in_tile(int l, int lim) {
 }
 
 // Periodic wrap with the reference migrate semantics; identical to the
-// oracle's wrap_coord (one-period fast paths are exact rewrites of fmodf).
+// oracle's wrap_coord (within a period of the box fmodf is one exact addition).
 __device__ __forceinline__ float wrap_coord(float v, float n) {
-    if (v >= n) {
-        v = (v < 2.0f * n) ? v - n : fmodf(v, n);
-    } else if (v < 0.0f) {
-        if (!(v > -n)) v = fmodf(v, n);
-        if (v < 0.0f) v += n;
+    float r = v >= n ? v - n : v;
+    r = v < 0.0f ? v + n : r;
+    if (!(v > -n && v < 2.0f * n)) {  // more than a period away, or not a number
+        r = v;
+        if (v >= n || v < 0.0f) r = fmodf(v, n);
+        if (r < 0.0f) r += n;
     }
-    if (v >= n) v = 0.0f;
-    return v;
+    return r >= n ? 0.0f : r;
 }
 
 __device__ __forceinline__ int cell_of(float x, float y, int nx, int ny) {
@@ -669,6 +669,75 @@ __device__ __forceinline__ void esk_emit(const EskShape& m, double cJx, double c
             if (v) add(2, k + 1, b + 1, v);
         }
     }
+}
+
+// The move geometry when both ends lie in cell (ib, jb) = floor(X0, Y0): the
+// shapes at the third node are exact zeros, DS at the second is -DS at the
+// first and the prefix sum P_1 (Q_1) is zero, so 2 + 2 + 4 contributions
+// remain of esk_emit's 21, each the same operations on the same values.  fx0,
+// fy0 (fx1, fy1) are the old (new) fractions, exact in FP32 for positions >= 0.
+struct EskCell {
+    double s0x0, s0y0, s1x0, s1y0;  // node-0 shapes 1 - f of the old and new position
+    double mx[2], my[2], dx, dy;    // node 0 and 1 means; node-0 difference
+};
+
+__device__ __forceinline__ EskCell esk_cell(double fx0, double fy0, double fx1, double fy1) {
+    EskCell m;
+    m.s0x0 = 1.0 - fx0;
+    m.s0y0 = 1.0 - fy0;
+    m.s1x0 = 1.0 - fx1;
+    m.s1y0 = 1.0 - fy1;
+    m.mx[0] = 0.5 * (m.s0x0 + m.s1x0);
+    m.my[0] = 0.5 * (m.s0y0 + m.s1y0);
+    m.mx[1] = 0.5 * ((1.0 - m.s0x0) + (1.0 - m.s1x0));
+    m.my[1] = 0.5 * ((1.0 - m.s0y0) + (1.0 - m.s1y0));
+    m.dx = m.s1x0 - m.s0x0;
+    m.dy = m.s1y0 - m.s0y0;
+    return m;
+}
+
+// esk_emit of such a move: add(q, k, b, v) with k, b in 1..2.  The caller
+// clamps: cJx, cJy = clamp_fix_f64 of esk_emit's, cz = clamp_fix_f64(cJz 16/12).
+template <class Add>
+__device__ __forceinline__ void esk_emit_cell(const EskCell& m, double cJx, double cJy, double cz,
+                                              Add&& add) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) add(0, 1, b + 1, fix_mul(cJx, m.dx * m.my[b]));
+#pragma unroll
+    for (int k = 0; k < 2; ++k) add(1, k + 1, 1, fix_mul(cJy, m.dy * m.mx[k]));
+    const double dy16 = (1.0 / 16.0) * m.dy;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        const double my12 = (12.0 / 16.0) * m.my[b], dyb = b ? -dy16 : dy16;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            add(2, k + 1, b + 1, fix_mul(cz, fma(k ? -m.dx : m.dx, dyb, m.mx[k] * my12)));
+    }
+}
+
+// Both ends of a move in one cell, at positions from which esk_cell's FP32
+// fractions are exact.  On a one-row grid esk_shape may take the periodic
+// image of a y move of more than half a cell (ny / 2): not this case.
+__device__ __forceinline__ bool esk_same_cell(float x0, float y0, float x1, float y1, float flx,
+                                              float fly, int nx, int ny) {
+    bool in = (flx == floorf(x1)) & (fly == floorf(y1)) & (fminf(flx, fly) >= 0.f);
+    if (nx == 1 || ny == 1) {
+        in = in && (nx > 1 || fabs((double)x1 - (double)x0) <= 0.5) &&
+             (ny > 1 || fabs((double)y1 - (double)y0) <= 0.5);
+    }
+    return in;
+}
+
+// a / b for an FP32 value b and its rounded reciprocal r = 1 / b: the product
+// a r is off by less than two units in the last place, and one residual (exact
+// by fma) corrects it.  The corrected quotient is off the true one by 2^-52 of
+// a unit before its rounding, while a quotient by a 24-bit divisor keeps 2^-25
+// of a unit away from every rounding boundary: the result is the correctly
+// rounded quotient (P. Markstein, IBM J. Res. Dev. 34, 1990), in 3 FP64
+// operations.
+__device__ __forceinline__ double div_by_f32(double a, double b, double r) {
+    const double q = a * r;
+    return fma(fma(-b, q, a), r, q);
 }
 
 // The dispatcher hands consecutive workgroup ids to the 8 XCDs in turn.  This

@@ -102,6 +102,80 @@ __device__ __forceinline__ void esk_emit(const EskMove& m, Add&& add) {
     }
 }
 
+// Moves that leave their cell, set aside by a wavefront in its own LDS slots
+// until cap of them fill (most of) a wavefront.  A move inside one cell has 8
+// of the 21 contributions and about a third of the arithmetic; moves that
+// leave theirs are a few percent, but nearly every wavefront has one, and
+// handled on the spot they would cost all 64 lanes the general stencil.
+// Every lane of the wavefront calls push and drain.
+struct MoveQueue {
+    static constexpr int kFloats = 6;  // LDS per slot
+    float* s;                          // this wavefront's slots, [6][cap]
+    int cap;
+    int cnt = 0;                       // wave-uniform
+
+    // body(x0, y0, x1, y1, uz, w) runs once per set-aside move
+    template <class Body>
+    __device__ __forceinline__ void push(bool want, float x0, float y0, float x1, float y1,
+                                         float uz, float w, Body&& body) {
+        unsigned long long m = __ballot(want);
+        while (m) {
+            const int pos = cnt + (int)__builtin_amdgcn_mbcnt_hi(
+                                      (unsigned)(m >> 32),
+                                      __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            const bool put = want && pos < cap;
+            if (put) {
+                s[pos] = x0;
+                s[cap + pos] = y0;
+                s[2 * cap + pos] = x1;
+                s[3 * cap + pos] = y1;
+                s[4 * cap + pos] = uz;
+                s[5 * cap + pos] = w;
+                want = false;
+            }
+            cnt = min(cap, cnt + (int)__popcll(m));
+            m = __ballot(want);
+            if (m) drain(body);
+        }
+    }
+
+    template <class Body>
+    __device__ __forceinline__ void drain(Body&& body) {
+        // the slots are this wavefront's own: its LDS accesses complete in
+        // program order, the fences keep the compiler to that order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int l = (int)(threadIdx.x & 63); l < cnt; l += 64)
+            body(s[l], s[cap + l], s[2 * cap + l], s[3 * cap + l], s[4 * cap + l],
+                 s[5 * cap + l]);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        cnt = 0;
+    }
+};
+
+// esk_emit for a move inside its cell (one-row grids: each column's rows
+// summed first, at row 1)
+template <bool ONE_ROW, class Add>
+__device__ __forceinline__ void esk_emit_cell(const dev::EskCell& m, double cJx, double cJy,
+                                              double cz, Add&& add) {
+    if constexpr (!ONE_ROW) {
+        dev::esk_emit_cell(m, cJx, cJy, cz, add);
+    } else {
+        unsigned long long col[3][3] = {};
+        dev::esk_emit_cell(m, cJx, cJy, cz,
+                           [&](int q, int k, int, unsigned long long v) { col[q][k] += v; });
+        add(0, 1, 1, col[0][1]);
+#pragma unroll
+        for (int k = 1; k < 3; ++k) {
+            add(1, k, 1, col[1][k]);
+            add(2, k, 1, col[2][k]);
+        }
+    }
+}
+
 __device__ __forceinline__ int wrap_local(int l, int n) {
     if (l < 0) l += n;
     else if (l >= n) l -= n;

@@ -167,6 +167,7 @@ struct PushArgs {
     unsigned int* guard;
     int n;
     double tnow;
+    double rdx, rdy;  // 1 / m.dx, 1 / m.dy
 };
 
 // what the current deposit needs of one pushed particle
@@ -174,6 +175,9 @@ struct PushOut {
     float x0, y0, x1, y1;  // the move (x1 before the periodic wrap)
     float uz;              // deposit velocity: uz / gamma (rel, walls) or uz
     float w;               // deposit weight (w wd for delta-f, else w)
+    float vx, vy, vz;      // the velocity to store
+    int col, row;          // of the gather (Fields6)
+    bool in;
 };
 
 // yee_advance_particle (include/pic/yee2d.hpp:145-302): staggered gather of
@@ -211,75 +215,103 @@ __device__ __forceinline__ float cic_mesh(const float* a, const Mesh& m, const C
 
 constexpr float kOx[4] = {0.5f, 0.f, 0.f, 0.5f}, kOy[4] = {0.f, 0.5f, 0.f, 0.5f};
 
+struct Fields6 {
+    float ex, ey, ez, bx, by, bz;
+    // of a window gather: the particle's cell in the window, and whether its
+    // stencils all lie inside
+    int col, row;
+    bool in;
+};
+
 // gathers straight from the mesh; staggering s: 0 (ex, by), 1 (ey, bx), 2 ez, 3 bz
 struct MeshGather {
     const Mesh& m;
-    __device__ __forceinline__ void two(int s, float x, float y, float& a, float& b) const {
-        const Cic c(x, y, kOx[s], kOy[s]);
-        a = cic_mesh(s == 0 ? m.ex : m.ey, m, c);
-        b = cic_mesh(s == 0 ? m.by : m.bx, m, c);
-    }
-    __device__ __forceinline__ float one(int s, float x, float y) const {
-        const Cic c(x, y, kOx[s], kOy[s]);
-        return cic_mesh(s == 2 ? m.ez : m.bz, m, c);
+    __device__ __forceinline__ void all(float x, float y, Fields6& f) const {
+        const Cic c0(x, y, kOx[0], kOy[0]), c1(x, y, kOx[1], kOy[1]);
+        f.ex = cic_mesh(m.ex, m, c0);
+        f.by = cic_mesh(m.by, m, c0);
+        f.ey = cic_mesh(m.ey, m, c1);
+        f.bx = cic_mesh(m.bx, m, c1);
+        f.ez = cic_mesh(m.ez, m, Cic(x, y, kOx[2], kOy[2]));
+        f.bz = cic_mesh(m.bz, m, Cic(x, y, kOx[3], kOy[3]));
     }
 };
 
-// gathers from a workgroup's LDS copy of the fields over the cells
-// [orgx, orgx + W) x [orgy, orgy + H) (periodically wrapped): planes of
-// float2 (ex, by), float2 (ey, bx), float ez, float bz.  A stencil that
-// leaves the window reads the mesh; the window holds the mesh's own values,
-// so both return the same bits.
+// gathers from a workgroup's LDS copy of the fields over the W x H cells from
+// (orgx, orgy) (periodically wrapped): planes of float2 (ex, by), float2
+// (ey, bx), float ez, float bz.  A stencil that leaves the window reads the
+// mesh; the window holds the mesh's own values, so both return the same bits.
+template <int W, int H>
 struct WindowGather {
     const float* s;
     const Mesh& m;
-    int orgx, orgy, W, H;
-    __device__ __forceinline__ bool local(const Cic& c, int& l) const {
-        int li = c.i0 - orgx, lj = c.j0 - orgy;
-        if ((unsigned)li > (unsigned)(W - 2)) li += li < 0 ? m.nx : -m.nx;
-        if ((unsigned)lj > (unsigned)(H - 2)) lj += lj < 0 ? m.ny : -m.ny;
-        l = lj * W + li;
-        return (unsigned)li <= (unsigned)(W - 2) && (unsigned)lj <= (unsigned)(H - 2);
+    int orgx, orgy;
+    // The four staggerings share two columns and two rows of corners: one
+    // test serves all of them.  Every lane reads the window (a stencil outside
+    // it a corner of it), so that the reads stay LDS instructions.
+    __device__ __forceinline__ void all(float x, float y, Fields6& f) const {
+        const Cic c0(x, y, kOx[0], kOy[0]), c1(x, y, kOx[1], kOy[1]), c2(x, y, kOx[2], kOy[2]),
+            c3(x, y, kOx[3], kOy[3]);
+        constexpr int R = W * H;
+        int ln = local(c2.i0 - orgx, W - 2, m.nx), rn = local(c2.j0 - orgy, H - 2, m.ny);
+        int lh = ln + (c3.i0 - c2.i0), rh = rn + (c3.j0 - c2.j0);
+        f.in = max((unsigned)ln, (unsigned)lh) <= (unsigned)(W - 2) &&
+               max((unsigned)rn, (unsigned)rh) <= (unsigned)(H - 2);
+        f.col = ln;
+        f.row = rn;
+        ln = f.in ? ln : 0;
+        lh = f.in ? lh : 0;
+        rn = f.in ? rn : 0;
+        rh = f.in ? rh : 0;
+        const int tn = rn * W, th = rh * W;
+        two(c0, tn + lh, f.ex, f.by);
+        two(c1, R + th + ln, f.ey, f.bx);
+        f.ez = one(c2, 4 * R + tn + ln);
+        f.bz = one(c3, 5 * R + th + lh);
+        if (!f.in) MeshGather{m}.all(x, y, f);
     }
-    __device__ __forceinline__ void two(int st, float x, float y, float& a, float& b) const {
-        const Cic c(x, y, kOx[st], kOy[st]);
-        int l;
-        if (!local(c, l)) {
-            a = cic_mesh(st == 0 ? m.ex : m.ey, m, c);
-            b = cic_mesh(st == 0 ? m.by : m.bx, m, c);
-            return;
-        }
-        const float2* p = reinterpret_cast<const float2*>(s) + st * W * H + l;
+    // l, or its periodic image where l leaves the window
+    __device__ __forceinline__ static int local(int l, int lim, int n) {
+        return l + (l < 0 ? n : (l > lim ? -n : 0));
+    }
+    __device__ __forceinline__ void two(const Cic& c, int l, float& a, float& b) const {
+        const float2* p = reinterpret_cast<const float2*>(s) + l;
         const float2 v00 = p[0], v10 = p[1], v01 = p[W], v11 = p[W + 1];
         a = c.mix(v00.x, v10.x, v01.x, v11.x);
         b = c.mix(v00.y, v10.y, v01.y, v11.y);
     }
-    __device__ __forceinline__ float one(int st, float x, float y) const {
-        const Cic c(x, y, kOx[st], kOy[st]);
-        int l;
-        if (!local(c, l)) return cic_mesh(st == 2 ? m.ez : m.bz, m, c);
-        const float* p = s + (st + 2) * W * H + l;
+    __device__ __forceinline__ float one(const Cic& c, int l) const {
+        const float* p = s + l;
         return c.mix(p[0], p[1], p[W], p[W + 1]);
     }
 };
 
-// One particle: the push updates u (and the delta-f weight) in place and
-// returns the move; the caller stores the positions.
+// a particle's values before the push
+struct PushIn {
+    float x, y, ux, uy, uz, w;
+};
+
+__device__ __forceinline__ PushIn load_particle(const PushArgs& a, int t) {
+    return {a.x[t], a.y[t], a.ux[t], a.uy[t], a.uz[t], a.w ? a.w[t] : a.w_uniform};
+}
+
+// One particle: the push updates the delta-f weight in place and
+// returns the move; the caller stores the positions and velocities.
 template <bool PLAIN, class Gather, bool NOPR = false>
 __device__ __forceinline__ void push_one(const PushArgs& a, const Mesh& m, const aw_run_params& rp,
-                                         int t, PushOut& o, const Gather& gat) {
+                                         int t, const PushIn& p, PushOut& o,
+                                         const Gather& gat) {
     // PLAIN: none of the pump, relativistic push, B0 profile, delta-f weights
     // or walls; NOPR: no pump or relativistic push (compile-time instances
     // without their registers)
     const bool pump = !PLAIN && !NOPR && rp.pump, rel = !PLAIN && !NOPR && rp.rel;
     const bool b0_prof = !PLAIN && rp.b0_prof, deltaf = !PLAIN && rp.deltaf;
     const int bnd_x = PLAIN ? 0 : rp.bnd_x;
-    const float x0 = a.x[t], y0 = a.y[t];
-    float Ex, Ey, dBx, dBy;
-    gat.two(0, x0, y0, Ex, dBy);
-    gat.two(1, x0, y0, Ey, dBx);
-    float Ez = gat.one(2, x0, y0);
-    const float dBz = gat.one(3, x0, y0);
+    const float x0 = p.x, y0 = p.y;
+    Fields6 f;
+    gat.all(x0, y0, f);
+    float Ex = f.ex, Ey = f.ey, Ez = f.ez;
+    const float dBx = f.bx, dBy = f.by, dBz = f.bz;
     if (pump && a.tnow < rp.pump_toff) {
         const double th = rp.pump_k0 * (double)x0 * (double)m.dx - rp.pump_w0 * a.tnow;
         const double r = ramp_of(a.tnow, rp.pump_trmp, rp.pump_toff);
@@ -287,7 +319,7 @@ __device__ __forceinline__ void push_one(const PushArgs& a, const Mesh& m, const
         Ey += (float)(-rp.pump_ey * sin(th) * r);
         Ez += (float)(rp.pump_ez * cos(th) * r);
     }
-    float ux = a.ux[t], uy = a.uy[t], uz = a.uz[t];
+    float ux = p.ux, uy = p.uy, uz = p.uz;
     const float uxo = ux, uyo = uy, uzo = uz;  // u^{n-1/2}
     const float qmh = (float)(rp.qm * 0.5 * rp.dt);
     ux = fmaf(qmh, Ex, ux);
@@ -358,11 +390,11 @@ __device__ __forceinline__ void push_one(const PushArgs& a, const Mesh& m, const
             wn = fminf(fmaxf((wd + (float)(rp.dt * rp.qm) * (1.f - wd) * S) * relax, lo), hi);
         }
         a.wd[t] = wn;
-        wdv = (a.w ? a.w[t] : a.w_uniform) * wn;
+        wdv = p.w * wn;
         if (a.wdep) a.wdep[t] = wdv;
     }
-    float x1 = x0 + (float)((double)(ux * gnew) * rp.dt / (double)m.dx);
-    const float y1 = y0 + (float)((double)(uy * gnew) * rp.dt / (double)m.dy);
+    float x1 = x0 + (float)dev::div_by_f32((double)(ux * gnew) * rp.dt, (double)m.dx, a.rdx);
+    const float y1 = y0 + (float)dev::div_by_f32((double)(uy * gnew) * rp.dt, (double)m.dy, a.rdy);
     float uxs = ux, uys = uy, uzs = uz;
     if (bnd_x) {  // specular walls at the domain ends (include/pic/yee2d.hpp:276-297)
         const float fnx = (float)m.nx;
@@ -386,12 +418,12 @@ __device__ __forceinline__ void push_one(const PushArgs& a, const Mesh& m, const
             }
         }
     }
-    a.ux[t] = uxs;
-    a.uy[t] = uys;
-    a.uz[t] = uzs;
+    o.vx = uxs;
+    o.vy = uys;
+    o.vz = uzs;
     // the current's uz/gamma is taken before the walls damp u
     const float uzd = (rel || bnd_x) ? uz * gnew : uzs;
-    const float wp = a.w ? a.w[t] : a.w_uniform;
+    const float wp = p.w;
     if (!(fabsf(uzd) <= a.ucap) || (a.w && !(fabsf(wp) <= a.wmax))) atomicOr(a.guard, 1u);
     o.x0 = x0;
     o.y0 = y0;
@@ -399,6 +431,9 @@ __device__ __forceinline__ void push_one(const PushArgs& a, const Mesh& m, const
     o.y1 = y1;
     o.uz = uzd;
     o.w = deltaf ? wdv : wp;
+    o.col = f.col;
+    o.row = f.row;
+    o.in = f.in;
 }
 
 // MaxwellSimulation's particle push (include/pic/yee2d.hpp:140-300), grid-
@@ -414,11 +449,14 @@ yee_push_kernel(PushArgs a, Mesh m, aw_run_params rp) {
     for (int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x; t < a.n;
          t += (int64_t)kThreads * gridDim.x) {
         PushOut o;
-        push_one<PLAIN, MeshGather, NOPR>(a, m, rp, (int)t, o, gat);
+        push_one<PLAIN, MeshGather, NOPR>(a, m, rp, (int)t, load_particle(a, (int)t), o, gat);
         a.x0[t] = o.x0;
         a.y0[t] = o.y0;
         a.x[t] = o.x1;
         a.y[t] = o.y1;
+        a.ux[t] = o.vx;
+        a.uy[t] = o.vy;
+        a.uz[t] = o.vz;
         if (a.vz) a.vz[t] = o.uz;
         if (a.wdep) a.wdep[t] = o.w;
     }
@@ -434,41 +472,85 @@ yee_push_kernel(PushArgs a, Mesh m, aw_run_params rp) {
 // touches HBM: the positions are stored wrapped, as the migrate does.
 struct PushTiles {
     const int32_t* off;  // ntiles + 1
-    const int32_t* idx;  // bin permutation (NULL: the particles are in tile order)
-    int ntx, tx, ty, D, W, H, bpt;  // field window: W = tx + 2 D + 2, H = ty + 2 D + 2
-    int JW, JH;                     // current window: tx + 2 A, ty + 2 A
+    const int32_t* idx;  // bin permutation (IDX; else the particles are in tile order)
+    int ntx, tx, ty, bpt;
 };
 
-// Register budgets, measured on the 156 M-particle eaw_case7 step: the
-// general instance at 4 waves per SIMD (128 VGPRs, 12 spilled) took 3.32 ms
-// against 3.81 ms at the compiler's 152 VGPRs (3 waves) and 4.08 ms at 5
-// waves (39 spilled); the plain instance at 6 waves (80 VGPRs, 4 spilled),
-// which is also as many as its 25 KB of LDS lets a CU hold, took 2.70 ms
-// against 3.04 ms at its own 91 VGPRs (5 waves).
-template <bool ONE_ROW, bool PLAIN>
+// The windows of a tile of up to T x T cells: fields with D cells of drift and the half-cell
+// stencils' extra column and row, the current with A nodes.  On a one-row
+// grid every row is the same one: the fields keep rows -1..1, the current
+// its one row (esk_emit's row 1).
+template <bool ONE_ROW>
+struct TileWindow {
+    static constexpr int T = 16, D = kPushApron, A = esk::kSortedApron;
+    static constexpr int W = T + 2 * D + 2, H = ONE_ROW ? 3 : T + 2 * D + 2, R = W * H;
+    static constexpr int JW = T + 2 * A, JH = ONE_ROW ? 4 : T + 2 * A, RJ = JW * JH;
+    static constexpr size_t kLds = 3 * RJ * sizeof(unsigned long long) + 6 * R * sizeof(float);
+};
+
+// Bound by VALU issue: 156 M particles of the oblique-whistler deck (625^2, 400
+// per cell) took 2275 us at 492 vector instructions a particle and 1632 us at
+// 332 (HBM: 40 B a particle, 1200 us).  What went: the 13 contributions of a
+// move that does not leave its cell which are zero, the FP64 divisions of the
+// move, one window test instead of four, and 64-bit addresses of particles in
+// tile order.  4 waves per SIMD (117 VGPRs) let the next particle's loads stay
+// in flight; 5 (96) spilled 18 registers and took 2135 us against 1846 us
+// before the addressing changed.
+using esk::MoveQueue;
+constexpr int kQueueSlots = 64;
+
+template <bool ONE_ROW, bool PLAIN, bool IDX>
 __global__ void __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(PLAIN ? 6 : 4, PLAIN ? 6 : 4)))
+__attribute__((amdgpu_waves_per_eu(4, 4)))
 yee_push_esk_tiles_kernel(PushArgs a, Mesh m, aw_run_params rp, PushTiles t, esk::EskArgs e,
                           unsigned long long* __restrict__ acc) {
     extern __shared__ unsigned long long s_mem[];
-    const int RJ = t.JW * t.JH, R = t.W * t.H;
+    using Win = TileWindow<ONE_ROW>;
+    constexpr int W = Win::W, R = Win::R, JW = Win::JW, JH = Win::JH, RJ = Win::RJ;
     unsigned long long* s_j = s_mem;                       // [3][JH][JW]
     float* s_f = reinterpret_cast<float*>(s_mem + 3 * RJ);  // field planes
+    MoveQueue queue{s_f + 6 * R + (threadIdx.x >> 6) * kQueueSlots * MoveQueue::kFloats, kQueueSlots};
     const int lb = dev::xcd_block(blockIdx.x, gridDim.x);
     const int tile = lb / t.bpt, part = lb % t.bpt;
     const int tx0 = (tile % t.ntx) * t.tx, ty0 = (tile / t.ntx) * t.ty;
-    const int orgx = tx0 - t.D - 1, orgy = ty0 - t.D - 1;
-    const int jorgx = tx0 - esk::kSortedApron, jorgy = ty0 - esk::kSortedApron;
+    const int orgx = tx0 - Win::D - 1, orgy = ONE_ROW ? -1 : ty0 - Win::D - 1;
+    const int jorgx = tx0 - Win::A, jorgy = ONE_ROW ? -1 : ty0 - Win::A;
+    const int beg = t.off[tile], end = t.off[tile + 1];
+    const int chunk = (end - beg + t.bpt - 1) / t.bpt;
+    const int r0 = beg + part * chunk, r1 = min(end, r0 + chunk);
+    if (r0 >= r1) return;
+    // Particle k of the wave-uniform first particle b (particles in tile order:
+    // a lane's offset from b is below kThreads), or particle k (IDX).
+    auto slot = [&](float* q, int b, int k) -> float& {
+        if constexpr (IDX) return q[k];
+        else return *reinterpret_cast<float*>(reinterpret_cast<char*>(q + b) + ((unsigned)k << 2));
+    };
+    // a particle's loads are in flight while the one before it is pushed (the
+    // first ones while the windows are filled); lanes past the end load the
+    // last particle and drop it
+    auto index = [&](int b) {
+        const int k = min((int)threadIdx.x, r1 - 1 - b);
+        if constexpr (IDX) return t.idx[b + k];
+        else return k;
+    };
+    auto fetch = [&](int b, int k) {
+        return PushIn{slot(a.x, b, k),  slot(a.y, b, k),  slot(a.ux, b, k),
+                      slot(a.uy, b, k), slot(a.uz, b, k), a.w ? slot(const_cast<float*>(a.w), b, k)
+                                                              : a.w_uniform};
+    };
+    auto after = [&](int b) { return min(b + kThreads, r1 - 1); };
+    int i = index(r0), inext = index(after(r0));
+    PushIn p = fetch(r0, i);
     float2* s2 = reinterpret_cast<float2*>(s_f);
     // (row, column) of a thread's cells advance by the stride without dividing
-    const int dr = kThreads / t.W, dc = kThreads % t.W;
-    int row = threadIdx.x / t.W, col = threadIdx.x % t.W;
+    constexpr int dr = kThreads / W, dc = kThreads % W;
+    int row = threadIdx.x / W, col = threadIdx.x % W;
     for (int l = threadIdx.x; l < R; l += kThreads) {
         const int g = dev::wrapfar(orgy + row, m.ny) * m.nx + dev::wrapfar(orgx + col, m.nx);
         row += dr;
         col += dc;
-        if (col >= t.W) {
-            col -= t.W;
+        if (col >= W) {
+            col -= W;
             ++row;
         }
         s2[l] = make_float2(m.ex[g], m.by[g]);
@@ -478,54 +560,97 @@ yee_push_esk_tiles_kernel(PushArgs a, Mesh m, aw_run_params rp, PushTiles t, esk
     }
     for (int c = threadIdx.x; c < 3 * RJ; c += kThreads) s_j[c] = 0ull;
     __syncthreads();
-    const WindowGather gat{s_f, m, orgx, orgy, t.W, t.H};
+    const WindowGather<W, Win::H> gat{s_f, m, orgx, orgy};
     double kc[3];
     esk::esk_coefs(e, kc);
     const int64_t nc = (int64_t)m.nx * m.ny;
-    const int beg = t.off[tile], end = t.off[tile + 1];
-    const int chunk = (end - beg + t.bpt - 1) / t.bpt;
-    const int r0 = beg + part * chunk, r1 = min(end, r0 + chunk);
-    for (int r = r0 + (int)threadIdx.x; r < r1; r += kThreads) {
-        const int i = t.idx ? t.idx[r] : r;
-        PushOut o;
-        push_one<PLAIN>(a, m, rp, i, o, gat);
-        a.x[i] = dev::wrap_coord(o.x1, (float)m.nx);
-        a.y[i] = dev::wrap_coord(o.y1, (float)m.ny);
+    const double qwu = e.qm * e.w_uniform;
+    const double cJxu = dev::clamp_fix_f64(-qwu * kc[0]), cJyu = dev::clamp_fix_f64(-qwu * kc[1]);
+    // a move that leaves its cell, or whose stencil leaves the window
+    auto general = [&](float x0, float y0, float x1, float y1, float uz, float w) {
         esk::EskMove mv;
-        esk::esk_prepare_v(e, o.x0, o.y0, o.x1, o.y1, o.uz, e.per_w ? (double)o.w : e.w_uniform,
-                           kc, mv);
+        esk::esk_prepare_v(e, x0, y0, x1, y1, uz, e.per_w ? (double)w : e.w_uniform, kc, mv);
         const int li = esk::wrap_local(mv.sh.ib - 1 - jorgx, m.nx);
         const int lj = esk::wrap_local(mv.sh.jb - 1 - jorgy, m.ny);
-        if (dev::in_tile(li, t.JW - 4) && dev::in_tile(lj, t.JH - 4)) {
-            const int base = lj * t.JW + li;
+        if (dev::in_tile(li, JW - 4) && dev::in_tile(lj, JH - 4)) {
+            const int base = lj * JW + li;
             esk::esk_emit<ONE_ROW>(mv, [&](int q, int k, int b, unsigned long long v) {
-                atomicAdd(&s_j[q * RJ + base + b * t.JW + k], v);
+                atomicAdd(&s_j[q * RJ + base + b * JW + k], v);
             });
         } else {
+            int gx[3], gy[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                gx[k] = dev::wrapfar(mv.sh.ib + k, m.nx);
+                gy[k] = dev::wrapfar(mv.sh.jb + k, m.ny) * m.nx;
+            }
             esk::esk_emit<ONE_ROW>(mv, [&](int q, int k, int b, unsigned long long v) {
-                atomicAdd(&acc[q * nc + (int64_t)dev::wrapfar(mv.sh.jb - 1 + b, m.ny) * m.nx +
-                               dev::wrapfar(mv.sh.ib - 1 + k, m.nx)],
-                          v);
+                atomicAdd(&acc[q * nc + (gy[b - 1] + gx[k - 1])], v);
             });
         }
+    };
+    // every lane stays to the end of the loop: the queue is the wavefront's
+    for (int base = r0; base < r1; base += kThreads) {
+        const bool valid = base + (int)threadIdx.x < r1;
+        const int bnext = after(base);
+        const PushIn pn = fetch(bnext, inext);
+        const int inext2 = index(after(bnext));
+        bool leaves = false;
+        PushOut o;
+        if (valid) {
+            push_one<PLAIN>(a, m, rp, IDX ? i : base + i, p, o, gat);
+            slot(a.x, base, i) = dev::wrap_coord(o.x1, (float)m.nx);
+            slot(a.y, base, i) = dev::wrap_coord(o.y1, (float)m.ny);
+            slot(a.ux, base, i) = o.vx;
+            slot(a.uy, base, i) = o.vy;
+            slot(a.uz, base, i) = o.vz;
+            // the field window's cells are the current window's: a stencil
+            // inside the one is inside the other
+            static_assert(Win::D + 2 == Win::A && Win::W - 2 == JW - 4);
+            const float flx = floorf(o.x0), fly = floorf(o.y0);
+            leaves = !(o.in && dev::esk_same_cell(o.x0, o.y0, o.x1, o.y1, flx, fly, m.nx,
+                                                  ONE_ROW ? 1 : m.ny));
+            if (!leaves) {
+                const dev::EskCell c =
+                    dev::esk_cell((double)(o.x0 - flx), (double)(o.y0 - fly),
+                                  (double)(o.x1 - flx), (double)(o.y1 - fly));
+                double qw = qwu, cJx = cJxu, cJy = cJyu;
+                if (e.per_w) {
+                    qw = e.qm * (double)o.w;
+                    cJx = dev::clamp_fix_f64(-qw * kc[0]);
+                    cJy = dev::clamp_fix_f64(-qw * kc[1]);
+                }
+                const double cz = dev::clamp_fix_f64(qw * (double)o.uz * kc[2] * (16.0 / 12.0));
+                unsigned long long* sj = s_j + (ONE_ROW ? 0 : o.row * JW) + o.col;
+                esk::esk_emit_cell<ONE_ROW>(c, cJx, cJy, cz,
+                                            [&](int q, int k, int b, unsigned long long v) {
+                                                atomicAdd(&sj[q * RJ + b * JW + k], v);
+                                            });
+            }
+        }
+        p = pn;
+        i = inext;
+        inext = inext2;
+        queue.push(leaves, o.x0, o.y0, o.x1, o.y1, o.uz, o.w, general);
     }
+    queue.drain(general);
     __syncthreads();
     // rows of the three components follow each other: (row, column) over
     // 3 JH rows, advanced by the stride without dividing
-    const int jdr = kThreads / t.JW, jdc = kThreads % t.JW;
-    int jrow = threadIdx.x / t.JW, jcol = threadIdx.x % t.JW;
+    const int jdr = kThreads / JW, jdc = kThreads % JW;
+    int jrow = threadIdx.x / JW, jcol = threadIdx.x % JW;
     for (int c = threadIdx.x; c < 3 * RJ; c += kThreads) {
         const unsigned long long v = s_j[c];
         if (v) {
-            const int q = jrow >= 2 * t.JH ? 2 : (jrow >= t.JH ? 1 : 0);
+            const int q = jrow >= 2 * JH ? 2 : (jrow >= JH ? 1 : 0);
             const int gx = dev::wrapfar(jorgx + jcol, m.nx);
-            const int gy = dev::wrapfar(jorgy + jrow - q * t.JH, m.ny);
+            const int gy = dev::wrapfar(jorgy + jrow - q * JH, m.ny);
             atomicAdd(&acc[q * nc + (int64_t)gy * m.nx + gx], v);
         }
         jrow += jdr;
         jcol += jdc;
-        if (jcol >= t.JW) {
-            jcol -= t.JW;
+        if (jcol >= JW) {
+            jcol -= JW;
             ++jrow;
         }
     }
@@ -1178,6 +1303,8 @@ struct aw_maxwell {
             a.wdep = !fused && rp.deltaf ? wdep.get() : nullptr;
             a.n = (int)p.n;
             a.tnow = tnow;
+            a.rdx = 1.0 / (double)m.dx;
+            a.rdy = 1.0 / (double)m.dy;
             // The current's fixed-point scale comes from bounds fixed before the
             // push: |uz/gamma| <= 2 max(1, c) (below c for the relativistic
             // push), |w| <= the run's largest weight, and |w wd| <= 8 |w|
@@ -1209,7 +1336,7 @@ struct aw_maxwell {
                         sorted_x = p.x;
                         next_sort = nstep + kRebinEvery;
                     }
-                    t.idx = sperm.get();
+                    t.idx = sperm.get();  // the kernel's IDX instance
                 } else if (nstep >= next_sort || sorted_n != p.n || sorted_x != p.x) {
                     tile_sort(p, df);
                     next_sort = nstep + rp.tile_sort;
@@ -1218,23 +1345,26 @@ struct aw_maxwell {
                 t.ntx = ctx->ntx;
                 t.tx = ctx->tx;
                 t.ty = ctx->ty;
-                t.D = kPushApron;
-                t.W = t.tx + 2 * t.D + 2;
-                t.H = t.ty + 2 * t.D + 2;
-                t.JW = t.tx + 2 * esk::kSortedApron;
-                t.JH = t.ty + 2 * esk::kSortedApron;
+                AW_REQUIRE(t.tx <= TileWindow<false>::T && t.ty <= TileWindow<false>::T,
+                           "the tile is larger than the push's windows");
                 t.bpt = tile_bpt(*ctx, p.n);
-                const size_t sh = (size_t)3 * t.JW * t.JH * sizeof(unsigned long long) +
-                                  (size_t)6 * t.W * t.H * sizeof(float);
+                const size_t sh =
+                    (g.ny == 1 ? TileWindow<true>::kLds : TileWindow<false>::kLds) +
+                    (size_t)(kThreads / 64) * kQueueSlots * MoveQueue::kFloats * sizeof(float);
                 AW_REQUIRE(sh <= ctx->lds_per_block, "the tile windows do not fit LDS");
                 const esk::EskArgs e = esk::setup(*ctx, nullptr, nullptr, p, rp.qm, rp.dt, stream,
                                                   ex);
                 const bool plain =
                     !(rp.pump || rp.rel || rp.b0_prof || rp.deltaf || rp.bnd_x);
-                auto kern = g.ny == 1 ? (plain ? yee_push_esk_tiles_kernel<true, true>
-                                               : yee_push_esk_tiles_kernel<true, false>)
-                                      : (plain ? yee_push_esk_tiles_kernel<false, true>
-                                               : yee_push_esk_tiles_kernel<false, false>);
+                auto pick = [&](auto one_row, auto idx) {
+                    constexpr bool R = decltype(one_row)::value, I = decltype(idx)::value;
+                    return plain ? yee_push_esk_tiles_kernel<R, true, I>
+                                 : yee_push_esk_tiles_kernel<R, false, I>;
+                };
+                using Y = std::true_type;
+                using N = std::false_type;
+                auto kern = g.ny == 1 ? (t.idx ? pick(Y{}, Y{}) : pick(Y{}, N{}))
+                                      : (t.idx ? pick(N{}, Y{}) : pick(N{}, N{}));
                 hipLaunchKernelGGL(kern,
                                    dim3(ctx->ntiles * t.bpt), dim3(kThreads), sh, stream, a, m, rp,
                                    t, e, ctx->jacc.get());

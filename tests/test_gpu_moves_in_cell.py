@@ -1,0 +1,51 @@
+"""GPU test of the split current deposit: moves that stay in their cell are
+deposited on the spot with the 8 contributions that are not zero, the others
+are set aside and take the general stencil (esk_device.hpp).  The tile-ordered
+Yee step does so; the unsorted one on a grid whose current fits LDS deposits
+every move with the general stencil.  Fields and particles must be the same
+bits at every share of moves that leave their cell, on one-row, one-column and
+ragged grids, with uniform and per-particle weights."""
+import numpy as np
+import pytest
+
+from arcwarden_amd import _lib as L
+from arcwarden_amd.maxwell import MaxwellSimulation
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(tile_sort, nx, ny, step, per_w, n, steps=3):
+    dx, dt = 0.5, 0.05
+    rp = L.run_params(dt=dt, qm=-1.0, eps0=1.0, c=6.0)
+    rp.B0[0], rp.B0[2], rp.tile_sort = 0.3, 0.2, tile_sort
+    rng = np.random.default_rng(nx * 1000 + ny)
+    st = {"x": rng.uniform(0, nx, n).astype(np.float32),
+          "y": rng.uniform(0, ny, n).astype(np.float32)}
+    # positions on cell edges and denormally close to the origin
+    st["x"][:64] = np.floor(st["x"][:64])
+    st["y"][32:96] = np.floor(st["y"][32:96])
+    st["x"][96:112], st["y"][112:128] = 1e-30, 1e-12
+    for k in ("ux", "uy", "uz"):  # at most `step` cells a step
+        st[k] = (rng.uniform(-1, 1, n) * step * dx / dt).astype(np.float32)
+    sim = MaxwellSimulation(L.grid(nx, ny, nx * dx, ny * dx), rp)
+    w = rng.uniform(0.5, 1.5, n).astype(np.float32) * (dx * dx / 16) if per_w else None
+    sim.set_particles(st, w=w, **({} if per_w else {"w_uniform": dx * dx / 16}))
+    for _ in range(steps):
+        sim.step()
+    sim.synchronize()
+    M, P = sim.mesh_flat(), sim.particles()
+    sim.close()
+    cols = np.stack([P[k] for k in ("x", "y", "ux", "uy", "uz")])
+    return M, cols[:, np.lexsort(cols[::-1])]
+
+
+@pytest.mark.parametrize("step", [0.0, 0.02, 0.5, 0.98])
+@pytest.mark.parametrize("nx,ny,per_w", [(48, 40, False), (33, 17, True), (300, 1, False),
+                                         (17, 1, True), (2, 40, False), (1, 24, False)])
+def test_split_deposit_matches_the_general_stencil(gpu, nx, ny, per_w, step):
+    n = max(5000, 20 * nx * ny) + 37
+    M0, P0 = _run(0, nx, ny, step, per_w, n)
+    M1, P1 = _run(1, nx, ny, step, per_w, n)
+    assert step == 0.0 or np.abs(M0[-3 * nx * ny:]).max() > 0
+    assert np.array_equal(M0, M1)
+    assert np.array_equal(P0, P1)
