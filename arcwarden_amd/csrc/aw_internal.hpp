@@ -301,6 +301,10 @@ void deposit_rho_fixed(aw_ctx& c, const aw_particles& p, double qm, int policy,
                        const int32_t* sorted_off, hipStream_t s,
                        unsigned long long* acc = nullptr);
 int tile_bpt(const aw_ctx& c, int64_t n);
+int balanced_bpt(const aw_ctx& c, int64_t n, size_t lds, int waves, int fixed);
+// Darwin kernels (darwin.hip): their workgroups per tile unless configured
+int em_push_bpt(const aw_ctx& c, int64_t n);
+int em_moments_bpt(const aw_ctx& c, int64_t n);
 
 // Spectral (spectral.hip)
 void solve_es_contig(aw_ctx& c, const float* rho, float* E2, double eps0, hipStream_t s);

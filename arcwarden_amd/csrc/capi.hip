@@ -58,9 +58,8 @@ void em_moments(aw_ctx& c, const aw_particles& p, const int32_t* off, const int3
 void em_dcu(aw_ctx& c, const aw_particles& p, const int32_t* off, const int32_t* idx,
             const float* const* F, unsigned long long* acc3, const float* c_dcu, int bpt,
             unsigned long long* strays, hipStream_t s, const EmBatch& b);
-int em_push(aw_ctx& c, const aw_particles& p, const int32_t* off, const int32_t* idx,
-            const float* const* F, unsigned long long* acc8, const float* cq, double qm,
-            double dt, int bpt, unsigned long long* strays, double* ke_part, hipStream_t s,
+int em_push(aw_ctx& c, const aw_particles& p, const int32_t* off, const float* const* F,
+            unsigned long long* acc8, const float* cq, double qm, double dt, int bpt, unsigned long long* strays, double* ke_part, hipStream_t s,
             bool esk, const EmBatch& b);
 void deposit_rho_j_amu(aw_ctx& c, const aw_particles& p, double qm, float* const out[8],
                        hipStream_t s);
@@ -176,7 +175,8 @@ struct aw_sim {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> prof_ev;
     double prof_ms = 0.0;
     int64_t prof_launches = 0;
-    int bpt = 0;
+    int bpt = 0;                           // fused push (ES or Darwin)
+    int bpt_dcu = 0, bpt_moments = 0;      // Darwin deposits
 
     // ---- spectral Darwin (field_model == AW_MODEL_DARWIN) ----
     bool em = false;
@@ -300,8 +300,8 @@ struct aw_sim {
         const int64_t nc = ncell(*ctx);
         const int R = runs;
         if (!moments_ready) {
-            em_moments(*ctx, particles(), tile_off.get(), nullptr, acc8.get(), cqd.get(), bpt,
-                       nullptr, s, batch(8 * nc));
+            em_moments(*ctx, particles(), tile_off.get(), nullptr, acc8.get(), cqd.get(),
+                       bpt_moments, nullptr, s, batch(8 * nc));
             j_staggered = false;
         }
         moments_ready = false;
@@ -326,7 +326,7 @@ struct aw_sim {
         fields6(ed3.get(), Fd);
         dcu_scale(Fd, nc, fmax_part.get(), dcu_abs, dcu_signed, umax, nullptr, cdcu.get(),
                   inv.get() + 8, s, R, 3 * nc, 5 * nc, 11);
-        em_dcu(*ctx, particles(), tile_off.get(), nullptr, Fd, acc3.get(), cdcu.get(), bpt,
+        em_dcu(*ctx, particles(), tile_off.get(), nullptr, Fd, acc3.get(), cdcu.get(), bpt_dcu,
                strays.get(), s, batch(3 * nc));
         convert_multi(acc3.get(), src.get() + 4 * nc, fin7, nc, 3, inv.get() + 8, s, R, 3 * nc,
                       11 * nc, 7 * nc, 11);
@@ -355,7 +355,7 @@ struct aw_sim {
         const float* Fp[6];
         fields6(e3.get(), Fp);
         const bool esk = cfg.current_deposit == AW_CURRENT_ESIRKEPOV;
-        const int nblk = em_push(*ctx, particles(), tile_off.get(), nullptr, Fp, acc8.get(),
+        const int nblk = em_push(*ctx, particles(), tile_off.get(), Fp, acc8.get(),
                                  cqd.get(), rp.qm, rp.dt, bpt, strays.get(),
                                  dump ? ke_part.get() : nullptr, s, esk, batch(8 * nc));
         j_staggered = esk;
@@ -469,11 +469,24 @@ struct aw_sim {
         if ((double)(v % kRangeFlag) > frac * (double)n * runs) sort_requested = true;
     }
 
+    // Workgroups per tile of the particle kernels: as given, or each kernel's own.
+    void set_bpt(int nbpt) {
+        bpt = bpt_dcu = bpt_moments = nbpt;
+        if (nbpt > 0) return;
+        if (cfg.field_model != AW_MODEL_DARWIN) {
+            bpt = tile_bpt(*ctx, n);
+            return;
+        }
+        bpt = em_push_bpt(*ctx, n);
+        bpt_dcu = tile_bpt(*ctx, n);
+        bpt_moments = em_moments_bpt(*ctx, n);
+    }
+
     // Tile geometry and workgroups per tile of the particle kernels.
     void apply_exec(int tile, int nbpt) {
         AW_HIP(hipStreamSynchronize(stream));
         set_ctx_tiles(*ctx, tile, tile);
-        bpt = nbpt > 0 ? nbpt : tile_bpt(*ctx, n);
+        set_bpt(nbpt);
         size_buffers();
     }
 
@@ -550,7 +563,7 @@ struct aw_sim {
                         fields6(e3.get(), F);
                         em_dcu(*ctx, dst, tile_off.get(), nullptr, F, acc3.get(), cdcu.get(), b,
                                strays.get(), s, EmBatch{});
-                        em_push(*ctx, dst, tile_off.get(), nullptr, F, acc8.get(), cqd.get(),
+                        em_push(*ctx, dst, tile_off.get(), F, acc8.get(), cqd.get(),
                                 rp.qm, rp.dt, b, strays.get(), nullptr, s, esk, EmBatch{});
                     } else {
                         push_deposit_es(*ctx, dst, tile_off.get(), Ex(), Ey(), rp,
@@ -1344,8 +1357,7 @@ static std::unique_ptr<aw_sim> finish_sim(std::unique_ptr<aw_sim> sim, int runs)
     sim->rho.resize((size_t)nc);
     sim->E.resize((size_t)2 * nc);
     sim->strays.resize(1);
-    sim->bpt = sim->cfg.blocks_per_tile > 0 ? sim->cfg.blocks_per_tile
-                                            : tile_bpt(*sim->ctx, sim->n);
+    sim->set_bpt(sim->cfg.blocks_per_tile);
     sim->size_buffers();
     sim->grid_part.resize(R * aw_sim::kGridPart);
     sim->diag_out.resize(R * 4 * sim->diag_cap);

@@ -14,7 +14,9 @@
 // All eight moments (rho, Jx, Jy, Jz, amu0..amu3) and the three dcu
 // components accumulate fixed-point int64 quanta: each contribution is the
 // FP32 product v*W rounded to an integer, v carrying the quantity's 2^S scale.
-#include "aw_internal.hpp"
+#include "esk_device.hpp"
+
+#include <algorithm>
 
 namespace aw {
 
@@ -48,6 +50,7 @@ struct EmArgs {
     double dxdt, dydt;           // dx/dt, dy/dt (Esirkepov current coefficients)
     unsigned long long* strays;
     double* ke_part;
+    int qslots;                  // slots of a wavefront's move queue (ESK)
     // uniform batch (EmBatch): run blockIdx.y offsets its pointers by these
     long long bp, be, bb, ba, bk;
     int bo;
@@ -104,6 +107,18 @@ __device__ __forceinline__ void moments8(const float cq[3], float mw, float ux, 
     v[7] = ba * (uz * uy);
 }
 
+// the NQ moment values, clamped for fix_mul; notes one out of range
+template <int NQ>
+__device__ __forceinline__ void fix_values(const float* v_in, double* v, unsigned int& nstray) {
+    float top = 0.f;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        top = fmaxf(top, fabsf(v_in[q]));
+        v[q] = (double)dev::clamp_fix_f32(v_in[q]);
+    }
+    if (top > kRangeLimit) nstray |= kRangeBit;
+}
+
 // Deposits v[q] for the q < NQ selected by MASK (grid q of the tile / global
 // accumulators): 4 CIC contributions rint(v[q] * W_k) per moment, with the
 // FP64 weights of cic_d (exact products) and one fma per contribution.
@@ -113,13 +128,7 @@ __device__ __forceinline__ void deposit_q(unsigned long long* s_acc, int R, int 
                                           int orgx, int orgy, const dev::CicD& d,
                                           const float* v_in, unsigned int& nstray) {
     double v[NQ];
-    bool over = false;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        over = over || fabsf(v_in[q]) > kRangeLimit;
-        v[q] = dev::clamp_fix_f64((double)v_in[q]);
-    }
-    if (over) nstray |= kRangeBit;
+    fix_values<NQ>(v_in, v, nstray);
     const int mi = local_index(d.i0, orgx, nx), mj = local_index(d.j0, orgy, ny);
     if (dev::in_tile(mi, W - 2) && dev::in_tile(mj, H - 2)) {
         const int b = mj * W + mi;
@@ -241,10 +250,14 @@ __device__ __forceinline__ void esk_deposit(const EmArgs& a, const Frame& f,
         });
     } else {
         unsigned long long* g = a.acc + (size_t)a.ncell;
+        int gx[3], gy[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            gx[k] = dev::wrapfar(m.ib + k, a.nx);
+            gy[k] = dev::wrapfar(m.jb + k, a.ny) * a.nx;
+        }
         dev::esk_emit(m, cJx, cJy, cJz, [&](int q, int k, int b, unsigned long long v) {
-            atomicAdd(&g[(size_t)q * a.ncell + (size_t)dev::wrapfar(m.jb - 1 + b, a.ny) * a.nx +
-                         dev::wrapfar(m.ib - 1 + k, a.nx)],
-                      v);
+            atomicAdd(&g[(size_t)q * a.ncell + (gy[b - 1] + gx[k - 1])], v);
         });
     }
 }
@@ -316,42 +329,27 @@ __global__ void __launch_bounds__(kThreads) dcu_kernel(EmArgs a) {
     if (nstray && a.strays) atomicAdd(a.strays, stray_word(nstray));
 }
 
-// One particle of em_push_kernel, its SoA values already loaded.
-template <bool PER_W, bool KE, bool ESK>
-__device__ __forceinline__ void em_one(const EmArgs& a, const Frame& f, const float4* fa,
-                                       const float2* fb, unsigned long long* s_acc,
-                                       const float cq[3], int k, float x, float y, float ux,
-                                       float uy, float uz, float mw, unsigned int& nstray,
-                                       double& ke) {
-    const dev::CicF s = dev::cic_f(x, y);
-    float e[3], b[3];
-    if (!gather6(a, f, fa, fb, s, e, b)) ++nstray;
-    dev::boris_full(a.qmh, e[0], e[1], e[2], b[0], b[1], b[2], ux, uy, uz);
-    const float xn = dev::wrap_coord(fmaf(ux, a.cx, x), (float)a.nx);
-    const float yn = dev::wrap_coord(fmaf(uy, a.cy, y), (float)a.ny);
-    a.x[k] = xn;
-    a.y[k] = yn;
-    a.ux[k] = ux;
-    a.uy[k] = uy;
-    a.uz[k] = uz;
-    if constexpr (KE)
-        ke += (PER_W ? (double)mw : 1.0) * ((double)ux * ux + (double)uy * uy + (double)uz * uz);
-    float v[8];
-    moments8(cq, mw, ux, uy, uz, v);
-    if constexpr (ESK) {
-        deposit_q<8, 0xF1u>(s_acc, f.R, f.W, f.H, a.acc, a.ncell, a.nx, a.ny, f.orgx, f.orgy,
-                            dev::cic_d(xn, yn), v, nstray);
-        esk_deposit(a, f, s_acc, x, y, xn, yn, uz, (double)cq[1] * (double)mw);
-    } else {
-        deposit_q<8>(s_acc, f.R, f.W, f.H, a.acc, a.ncell, a.nx, a.ny, f.orgx, f.orgy,
-                     dev::cic_d(xn, yn), v, nstray);
-    }
-}
+// Moves that leave their cell wait in LDS (esk_device.hpp): as many slots as
+// the 16x16-cell tile leaves of a quarter of a CU's LDS (fewer where a larger
+// tile leaves less).
+using esk::MoveQueue;
+constexpr int kQueueSlots = 20;
 
-// ESK: the current of the next state
-// is the Esirkepov current of this step's move (staggered Jx, Jy), not the
-// CIC current at x^{n+1}; rho and amu stay CIC at x^{n+1}.  Two particles
-// per thread per iteration, both loaded before either is pushed.
+struct EmIn {
+    float x, y, ux, uy, uz, w;
+};
+
+// E, B gathered at x^n, Boris, move, wrap and the eight moments of the new
+// state.  ESK: the current is the Esirkepov current of this step's move
+// (staggered Jx, Jy), not the CIC current at x^{n+1}; rho and amu stay CIC at
+// x^{n+1}.  A move inside one cell (nearly all of them) has both on the same
+// four nodes: 20 + 8 contributions where the general stencil has 20 + 21.
+// Particle k of the uniform first particle `base` keeps a lane's offset below
+// 32 bits; the next iteration's loads are in flight while this one's particle
+// is pushed.  16.8 M particles (512x128, vth 0.019 cells a step), ESK: 325 ->
+// 286 us.  It is bound by LDS: a particle's 28 atomics take 14 cycles a
+// wavefront at random cells, its eight gather reads 93, 210 us in all
+// (HBM: 40 B a particle, 130 us).
 template <bool PER_W, bool KE, bool ESK>
 __global__ void __launch_bounds__(kThreads) em_push_kernel(EmArgs a) {
     select_run(a);
@@ -361,29 +359,92 @@ __global__ void __launch_bounds__(kThreads) em_push_kernel(EmArgs a) {
     unsigned long long* s_acc = smem;
     float4* fa = reinterpret_cast<float4*>(smem + kNq * f.R);
     float2* fb = reinterpret_cast<float2*>(fa + f.R);
+    MoveQueue queue{reinterpret_cast<float*>(fb + f.R) +
+                        (threadIdx.x >> 6) * a.qslots * MoveQueue::kFloats,
+                    a.qslots};
+    auto slot = [&](float* q, int b, int k) -> float& {
+        return *reinterpret_cast<float*>(reinterpret_cast<char*>(q + b) + ((unsigned)k << 2));
+    };
+    auto fetch = [&](int b) {  // lanes past the end load the last particle and drop it
+        const int k = min((int)threadIdx.x, f.r1 - 1 - b);
+        return EmIn{slot(a.x, b, k),  slot(a.y, b, k),  slot(a.ux, b, k), slot(a.uy, b, k),
+                    slot(a.uz, b, k), PER_W ? slot(const_cast<float*>(a.w), b, k) : 1.0f};
+    };
+    EmIn p{};
+    if (f.r0 < f.r1) p = fetch(f.r0);
     for (int c = threadIdx.x; c < kNq * f.R; c += kThreads) s_acc[c] = 0ull;
     load_fields(a, f, fa, fb);
     __syncthreads();
     unsigned int nstray = 0;
     double ke = 0.0;
     const float cq[3] = {a.cq[0], a.cq[1], a.cq[2]};
-    int r = f.r0 + (int)threadIdx.x;
-    for (; r + kThreads < f.r1; r += 2 * kThreads) {
-        const int k0 = a.idx ? a.idx[r] : r;
-        const int k1 = a.idx ? a.idx[r + kThreads] : r + kThreads;
-        const float x0 = a.x[k0], y0 = a.y[k0], ux0 = a.ux[k0], uy0 = a.uy[k0], uz0 = a.uz[k0];
-        const float x1 = a.x[k1], y1 = a.y[k1], ux1 = a.ux[k1], uy1 = a.uy[k1], uz1 = a.uz[k1];
-        const float w0 = PER_W ? a.w[k0] : 1.0f, w1 = PER_W ? a.w[k1] : 1.0f;
-        em_one<PER_W, KE, ESK>(a, f, fa, fb, s_acc, cq, k0, x0, y0, ux0, uy0, uz0, w0,
-                                    nstray, ke);
-        em_one<PER_W, KE, ESK>(a, f, fa, fb, s_acc, cq, k1, x1, y1, ux1, uy1, uz1, w1,
-                                    nstray, ke);
+    // the J coefficient (Jx = -cj dx/dt .., Jy = -cj dy/dt .., Jz = cj uz ..)
+    const double cju = (double)cq[1];
+    const double cJxu = dev::clamp_fix_f64(-cju * a.dxdt), cJyu = dev::clamp_fix_f64(-cju * a.dydt);
+    auto general = [&](float x0, float y0, float x1, float y1, float uz, float w) {
+        esk_deposit(a, f, s_acc, x0, y0, x1, y1, uz, (double)cq[1] * (double)w);
+    };
+    for (int base = f.r0; base < f.r1; base += kThreads) {
+        const bool valid = base + (int)threadIdx.x < f.r1;
+        const EmIn pn = fetch(min(base + kThreads, f.r1 - 1));
+        bool leaves = false;
+        float xn = 0.f, yn = 0.f, uz = 0.f;
+        if (valid) {
+            float ux = p.ux, uy = p.uy;
+            uz = p.uz;
+            const dev::CicF s = dev::cic_f(p.x, p.y);
+            float e[3], b[3];
+            if (!gather6(a, f, fa, fb, s, e, b)) ++nstray;
+            dev::boris_full(a.qmh, e[0], e[1], e[2], b[0], b[1], b[2], ux, uy, uz);
+            xn = dev::wrap_coord(fmaf(ux, a.cx, p.x), (float)a.nx);
+            yn = dev::wrap_coord(fmaf(uy, a.cy, p.y), (float)a.ny);
+            const int k = (int)threadIdx.x;
+            slot(a.x, base, k) = xn;
+            slot(a.y, base, k) = yn;
+            slot(a.ux, base, k) = ux;
+            slot(a.uy, base, k) = uy;
+            slot(a.uz, base, k) = uz;
+            if constexpr (KE)
+                ke += (PER_W ? (double)p.w : 1.0) *
+                      ((double)ux * ux + (double)uy * uy + (double)uz * uz);
+            float v[8];
+            moments8(cq, p.w, ux, uy, uz, v);
+            const dev::CicD d = dev::cic_d(xn, yn);
+            if constexpr (ESK) {
+                // rho and amu of every particle, then J of the moves inside a cell
+                deposit_q<8, 0xF1u>(s_acc, f.R, f.W, f.H, a.acc, a.ncell, a.nx, a.ny, f.orgx,
+                                    f.orgy, d, v, nstray);
+                const int mi = local_index(d.i0, f.orgx, a.nx),
+                          mj = local_index(d.j0, f.orgy, a.ny);
+                leaves = !(dev::esk_same_cell(p.x, p.y, xn, yn, floorf(p.x), floorf(p.y), a.nx,
+                                              a.ny) &&
+                           dev::in_tile(mi, f.W - 2) && dev::in_tile(mj, f.H - 2));
+                if (!leaves) {
+                    const dev::EskCell c = dev::esk_cell(
+                        (double)p.x - (double)d.i0, (double)p.y - (double)d.j0,
+                        (double)xn - (double)d.i0, (double)yn - (double)d.j0);
+                    double cj = cju, cJx = cJxu, cJy = cJyu;
+                    if constexpr (PER_W) {
+                        cj = (double)cq[1] * (double)p.w;
+                        cJx = dev::clamp_fix_f64(-cj * a.dxdt);
+                        cJy = dev::clamp_fix_f64(-cj * a.dydt);
+                    }
+                    const double cz = dev::clamp_fix_f64(cj * (double)uz * (16.0 / 12.0));
+                    unsigned long long* sj = s_acc + f.R + mj * f.W + mi;
+                    dev::esk_emit_cell(c, cJx, cJy, cz,
+                                       [&](int q, int k, int b, unsigned long long t) {
+                                           atomicAdd(&sj[q * f.R + (b - 1) * f.W + (k - 1)], t);
+                                       });
+                }
+            } else {
+                deposit_q<8>(s_acc, f.R, f.W, f.H, a.acc, a.ncell, a.nx, a.ny, f.orgx, f.orgy, d,
+                             v, nstray);
+            }
+        }
+        if constexpr (ESK) queue.push(leaves, p.x, p.y, xn, yn, uz, p.w, general);
+        p = pn;
     }
-    if (r < f.r1) {
-        const int k = a.idx ? a.idx[r] : r;
-        em_one<PER_W, KE, ESK>(a, f, fa, fb, s_acc, cq, k, a.x[k], a.y[k], a.ux[k],
-                                    a.uy[k], a.uz[k], PER_W ? a.w[k] : 1.0f, nstray, ke);
-    }
+    if constexpr (ESK) queue.drain(general);
     __shared__ double s_ke[kThreads / 64];
     if constexpr (KE) {
         for (int o = 32; o > 0; o >>= 1) ke += __shfl_down(ke, o, 64);
@@ -716,6 +777,17 @@ static EmArgs em_args(aw_ctx& c, const aw_particles& p, const int32_t* off, cons
     return a;
 }
 
+static size_t tile_nodes(const aw_ctx& c) {
+    return (size_t)(c.tx + 2 * c.apron + 1) * (c.ty + 2 * c.apron + 1);
+}
+// the moments' and the push's accumulators (and fields) per node of the tile
+int em_push_bpt(const aw_ctx& c, int64_t n) {
+    return balanced_bpt(c, n, tile_nodes(c) * 88, 4, 3);
+}
+int em_moments_bpt(const aw_ctx& c, int64_t n) {
+    return balanced_bpt(c, n, tile_nodes(c) * 64, 8, 3);
+}
+
 static void set_batch(EmArgs& a, const EmBatch& b) {
     a.bp = b.pstride;
     a.be = b.estride;
@@ -758,14 +830,20 @@ void em_dcu(aw_ctx& c, const aw_particles& p, const int32_t* off, const int32_t*
 
 // esk: the J moments of acc8 are the Esirkepov current of the move (staggered
 // Jx, Jy).
-int em_push(aw_ctx& c, const aw_particles& p, const int32_t* off, const int32_t* idx,
-            const float* const* F, unsigned long long* acc8, const float* cq, double qm,
+int em_push(aw_ctx& c, const aw_particles& p, const int32_t* off, const float* const* F,
+            unsigned long long* acc8, const float* cq, double qm,
             double dt, int bpt, unsigned long long* strays, double* ke_part, hipStream_t s,
             bool esk, const EmBatch& b) {
     if (p.n == 0) return 0;
-    EmArgs a = em_args(c, p, off, idx, F, acc8, cq, nullptr, qm, dt, bpt, strays, ke_part);
+    EmArgs a = em_args(c, p, off, nullptr, F, acc8, cq, nullptr, qm, dt, bpt, strays, ke_part);
     set_batch(a, b);
-    const size_t sh = (size_t)a.W * a.H * (8 * 8 + 16 + 8);
+    size_t sh = (size_t)a.W * a.H * (8 * 8 + 16 + 8);
+    if (esk) {
+        constexpr size_t slot = (kThreads / 64) * MoveQueue::kFloats * sizeof(float);
+        const size_t left = c.lds_per_block > sh ? c.lds_per_block - sh : 0;
+        a.qslots = (int)std::clamp<size_t>(left / slot, 1, kQueueSlots);
+        sh += a.qslots * slot;
+    }
     AW_REQUIRE(sh <= c.lds_per_block, "tile too large for the LDS of the EM push");
     const int nblk = c.ntiles * bpt;
     const bool pw = p.w != nullptr, ke = ke_part != nullptr;
@@ -875,7 +953,7 @@ void deposit_rho_j_amu(aw_ctx& c, const aw_particles& p, double qm, float* const
     bin_particles(c, p, s);
     measure_scales(c, p, qm, s);
     em_moments(c, p, c.sort.bin_off.get(), c.sort.bin_perm.get(), e.acc.get(), e.cq.get(),
-               tile_bpt(c, p.n), nullptr, s, EmBatch{});
+               em_moments_bpt(c, p.n), nullptr, s, EmBatch{});
     Out8 o{};
     for (int q = 0; q < 8; ++q) o.o[q] = out[q];
     convert_add_kernel<<<blocks_for(nc), kThreads, 0, s>>>(e.acc.get(), o, (int)nc, 8, e.inv.get());

@@ -217,6 +217,36 @@ int tile_bpt(const aw_ctx& c, int64_t n) {
     return bpt;
 }
 
+// tile_bpt for the kernels whose workgroups are few per CU (LDS windows,
+// registers).  A launch runs in rounds of as many workgroups as the chip holds
+// at once, each as long as a workgroup's windows (`fixed`, in iterations of one
+// particle per lane) plus its particles, so a little over a whole number of
+// rounds wastes most of one; past six rounds the workgroups finish out of step
+// and tile_bpt's share stands (156 M Yee particles: 1632 us, 1657 us with as few
+// workgroups as this would take).  lds: a workgroup's LDS; waves: the kernel's
+// waves per SIMD.  The relativistic Yee push of 0.98 M particles on 250x130 went
+// from 1152 workgroups to 1008 and from 38.9 to 34.3 us, the Darwin moments of
+// 1.6 M on 128x128 from 1664 to 1280 and from 96 to 61 us.
+int balanced_bpt(const aw_ctx& c, int64_t n, size_t lds, int waves, int fixed) {
+    const double per_tile = (double)n / std::max(1, c.ntiles);
+    const int per_cu = (int)std::clamp<size_t>(c.lds_per_block / std::max<size_t>(1, lds), 1,
+                                               (size_t)waves);
+    const double slots = (double)per_cu * std::max(1, c.num_cu);
+    int best = tile_bpt(c, n);
+    if ((double)c.ntiles * best > 6.0 * slots) return best;
+    double best_cost = 0.0;
+    for (int b = 1; b <= 64; ++b) {
+        if (b > 1 && per_tile / b < kThreads) break;
+        const double rounds = std::ceil((double)c.ntiles * b / slots);
+        const double cost = rounds * (fixed + std::ceil(per_tile / b / kThreads));
+        if (b == 1 || cost < best_cost) {
+            best = b;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
 // Accumulates rho of p into c.acc (fixed point).  sorted_off != nullptr:
 // particles are physically tile-sorted with those offsets (tiles policy,
 // direct reads).  policy BINNED without offsets bins first (stable).

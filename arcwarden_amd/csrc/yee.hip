@@ -1347,11 +1347,11 @@ struct aw_maxwell {
                 t.ty = ctx->ty;
                 AW_REQUIRE(t.tx <= TileWindow<false>::T && t.ty <= TileWindow<false>::T,
                            "the tile is larger than the push's windows");
-                t.bpt = tile_bpt(*ctx, p.n);
                 const size_t sh =
                     (g.ny == 1 ? TileWindow<true>::kLds : TileWindow<false>::kLds) +
                     (size_t)(kThreads / 64) * kQueueSlots * MoveQueue::kFloats * sizeof(float);
                 AW_REQUIRE(sh <= ctx->lds_per_block, "the tile windows do not fit LDS");
+                t.bpt = balanced_bpt(*ctx, p.n, sh, 4, 3);
                 const esk::EskArgs e = esk::setup(*ctx, nullptr, nullptr, p, rp.qm, rp.dt, stream,
                                                   ex);
                 const bool plain =
