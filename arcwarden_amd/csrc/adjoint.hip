@@ -673,10 +673,8 @@ struct aw_adjoint {
 
     // rho^n (in ctx->acc) -> rho, E2 = [Ex | Ey] (default: E); acc cleared
     void solve_current(float* E2 = nullptr) {
-        ctx->rin.reserve((size_t)ncell(*ctx));
-        fix_to_float_add(ctx->acc.get(), rho.get(), ncell(*ctx), ctx->fix_log2, true, stream, true,
-                         strays.get(), ctx->rin.get(), 1, nullptr, ctx->rho_base);
-        solve_es_contig(*ctx, ctx->rin.get(), E2 ? E2 : E.get(), rp.eps0, stream);
+        convert_solve_es(*ctx, ctx->acc.get(), rho.get(), E2 ? E2 : E.get(), rp.eps0, strays.get(),
+                         stream);
     }
 
     // up to four arrays of n floats, one launch
@@ -796,6 +794,15 @@ struct aw_adjoint {
             AW_LAUNCH_CHECK();
         } else {
             copy_words(lE0.get(), lEf.get(), (size_t)2 * nc * sizeof(float));
+        }
+        if (ctx->own_fft) {
+            static_assert(kBoundSlots == kSpecSlots && kSlotStride == kSpecSlotStride);
+            SpecSrc in;
+            in.in = lEf.get();
+            SpecDst out;
+            out.out = lrho.get();
+            spec_solve_es_adj(*ctx, in, out, rp.eps0, bd.get()->rmax, s);
+            return;
         }
         ctx->ktmp.reserve((size_t)6 * nk);
         float2* ak = reinterpret_cast<float2*>(ctx->ktmp.get());

@@ -161,6 +161,17 @@ inline BorisConsts boris_make(double qm, double dt_eff, const float B0[3], bool 
 // context
 // ---------------------------------------------------------------------------
 
+// A line transform (fft_device.hpp): the radices of its passes, a byte each.
+// Kernel arguments lie in host memory and a kernel waits about a microsecond
+// for each line of them that it reads late, so the plan is two words.
+struct FftLine {
+    static constexpr int kMaxPass = 8;
+    int n = 0, npass = 0;
+    unsigned long long radices = 0;
+    int ntw = 0;                  // twiddles the passes read: exp(-2 pi i k / n), k < ntw
+    const double2* tw = nullptr;
+};
+
 // Field-combination pointers: E = (E_L + E_T) + pump; ET[0] null means E_L + pump.
 struct FormE {
     float* E[3];
@@ -210,9 +221,12 @@ struct aw_ctx {
     long long rho_base = 0;
     int device = 0, num_cu = 0;
     size_t lds_per_block = 0;
-    // rocFFT
+    // the solves' own transforms (fft.hip) where the grid allows them
+    bool own_fft = false;
+    aw::FftLine fx, fy;
+    aw::DevBuf<double2> fft_tw;
     rocfft_plan r2c = nullptr, c2r = nullptr, c2r2 = nullptr;
-    rocfft_plan r2c2 = nullptr, r2c3 = nullptr, c2r3 = nullptr;
+    rocfft_plan r2c2 = nullptr, c2r3 = nullptr;
     rocfft_plan r2c4 = nullptr, r2c7 = nullptr, c2r5 = nullptr;  // Darwin batches
     rocfft_plan r2cB = nullptr, c2rB = nullptr;                  // ensemble batches
     int fft_batch = 0;
@@ -306,6 +320,69 @@ int balanced_bpt(const aw_ctx& c, int64_t n, size_t lds, int waves, int fixed);
 int em_push_bpt(const aw_ctx& c, int64_t n);
 int em_moments_bpt(const aw_ctx& c, int64_t n);
 
+// The external pump wave (include/pic/pump.hpp:34-47).
+struct PumpArgs {
+    int on;
+    double ex, ey, ez, k0, w0, trmp, toff, t, dx;
+};
+PumpArgs pump_args(const aw_grid& g, const aw_run_params& rp, double t);
+
+// Solves on the library's own transforms (fft.hip), which fuse the fixed-point
+// conversion before them and the field combination after them; only where
+// own_fft.  A SpecSrc describes the input grids (run r of a batch at r *_rs): fixed-point accumulators acc[q], converted as convert_multi does
+// (out[q] receives the FP32 grid, acc is cleared, the baseline is taken off
+// the transform's input only), or FP32 grids in.
+struct SpecSrc {
+    // grids q < split from acc + q nc, the others from acc2 + (q - split) nc
+    unsigned long long *acc = nullptr, *acc2 = nullptr;
+    long long acc_rs = 0, acc2_rs = 0;
+    int split = 7;
+    float* out = nullptr;       // the FP32 grid of q at out + out_at(q) nc
+    long long out_rs = 0;
+    const double* inv = nullptr;  // device scales, inv[inv_at(q)]; null: inv0
+    int inv_rs = 0, inv_a = 0, inv_b = 0, out_a = 0, out_b = 0;  // _at(q) = q + (q < split ? a : b)
+    double inv0 = 0.0;
+    const long long* base = nullptr;  // of grid 0, per cell (base_cell) or run
+    int base_cell = 0;
+    long long base_val = 0;
+    const float* in = nullptr;  // FP32 grids, contiguous
+    long long in_rs = 0;
+    unsigned long long* counter = nullptr;  // ncounter counters to clear
+    int ncounter = 0;
+};
+// The output grids, and what is formed from them on the way out:
+// E = E_L + pump with the maxima of |E| and |B| per workgroup (kFormEl: out =
+// [ELx|ELy|Bx|By|Bz]), or E = E_L + E_T + pump (kFormEt).
+struct SpecDst {
+    enum Form { kPlain, kFormEl, kFormEt };
+    float *out = nullptr, *out1 = nullptr;  // grid 0; grids 1.. contiguous
+    long long out_rs = 0;
+    Form form = kPlain;
+    float* e = nullptr;
+    long long e_rs = 0;
+    const float* el = nullptr;
+    long long el_rs = 0;
+    PumpArgs pump{};
+    float* part = nullptr;  // kFormEl: maxima, 2 spec_blocks(5) floats per run
+};
+// rho of the fixed-point accumulator acc (cleared) and its field: rho and
+// E2 = [Ex | Ey], the run's mean charge density left out of the transform
+void convert_solve_es(aw_ctx& c, unsigned long long* acc, float* rho, float* E2, double eps0,
+                      unsigned long long* counter, hipStream_t s);
+void init_own_fft(aw_ctx& c);
+int spec_blocks(const aw_ctx& c, int nq);
+void spec_solve_es(aw_ctx& c, const SpecSrc& in, const SpecDst& out, double eps0, int runs,
+                   hipStream_t s);
+// rmax: kSpecSlots slots, kSpecSlotStride words apart, whose largest receives
+// the largest |Re| + |Im| of the output's modes (FP32 bit patterns)
+constexpr int kSpecSlots = 64, kSpecSlotStride = 32;
+void spec_solve_es_adj(aw_ctx& c, const SpecSrc& in, const SpecDst& out, double eps0,
+                       unsigned int* rmax, hipStream_t s);
+void spec_solve_elb(aw_ctx& c, const SpecSrc& in, const SpecDst& out, double eps0, double cl,
+                    const float B0[3], bool stag, int runs, hipStream_t s);
+void spec_solve_et(aw_ctx& c, const SpecSrc& in, const SpecDst& out, double eps0, double cl,
+                   double n0, int runs, hipStream_t s);
+
 // Spectral (spectral.hip)
 void solve_es_contig(aw_ctx& c, const float* rho, float* E2, double eps0, hipStream_t s);
 void enable_batch_fft(aw_ctx& c, int batch);
@@ -371,6 +448,24 @@ __device__ __forceinline__ int wrapfar(int i, int n) {
 __device__ __forceinline__ void wrap_pair(int i, int n, int& a, int& b) {
     a = wrapfar(i, n);
     b = (a + 1 == n) ? 0 : a + 1;
+}
+
+__device__ __forceinline__ double pump_ramp(double t, double trmp, double toff) {
+    if (t >= toff) return 0.0;
+    if (t < trmp) return t / trmp;
+    if (t > toff - trmp) return (toff - t) / trmp;
+    return 1.0;
+}
+
+// the pump field of column i: E (the caller's FP32 addends)
+__device__ __forceinline__ void pump_at(const PumpArgs& p, int i, float& ex, float& ey, float& ez) {
+    const double x = i * p.dx;
+    const double th = p.k0 * x - p.w0 * p.t;
+    const double r = pump_ramp(p.t, p.trmp, p.toff);
+    const double ct = cos(th), st = sin(th);
+    ex = (float)(p.ex * ct * r);
+    ey = (float)(-p.ey * st * r);
+    ez = (float)(p.ez * ct * r);
 }
 
 // Max over the workgroup of (a, b), for workgroups of up to 1024 threads in
@@ -724,7 +819,7 @@ __device__ __forceinline__ void esk_emit_cell(const EskCell& m, double cJx, doub
 // image of a y move of more than half a cell (ny / 2): not this case.
 __device__ __forceinline__ bool esk_same_cell(float x0, float y0, float x1, float y1, float flx,
                                               float fly, int nx, int ny) {
-    bool in = (flx == floorf(x1)) & (fly == floorf(y1)) & (fminf(flx, fly) >= 0.f);
+    bool in = flx == floorf(x1) && fly == floorf(y1) && fminf(flx, fly) >= 0.f;
     if (nx == 1 || ny == 1) {
         in = in && (nx > 1 || fabs((double)x1 - (double)x0) <= 0.5) &&
              (ny > 1 || fabs((double)y1 - (double)y0) <= 0.5);

@@ -75,6 +75,9 @@ void form_e(const FormE& f, const aw_grid& g, const aw_run_params& rp, double t,
 void dcu_scale(const float* const* F, int64_t ncell, float* part, double coef_abs,
                double coef_signed, double umax, const double* dev, float* c_dcu, double* inv_dcu,
                hipStream_t s, int runs, long long sE, long long sB, int si);
+void dcu_scale_parts(const float* part, int nb, double coef_abs, double coef_signed, double umax,
+                     const double* dev, float* c_dcu, double* inv_dcu, hipStream_t s, int runs,
+                     int si);
 
 void check_grid(const aw_grid* g) {
     AW_REQUIRE(g != nullptr, "grid is NULL");
@@ -235,14 +238,15 @@ struct aw_sim {
         acc8.resize(R * 8 * nc);
         acc3.resize(R * 3 * nc);
         src.resize(R * 11 * nc);
-        fftin.resize(R * 11 * nc);  // [run][4] R2C inputs, then [run][7]
+        if (!ctx->own_fft) fftin.resize(R * 11 * nc);  // [run][4] R2C inputs, then [run][7]
         elb.resize(R * 5 * nc);
         et.resize(R * 3 * nc);
         e3.resize(R * 3 * nc);
         ed3.resize(R * 3 * nc);
         inv.resize(R * 11);
         cdcu.resize(R);
-        fmax_part.resize(R * (size_t)dcu_part_capacity());
+        fmax_part.resize(R * (size_t)std::max(dcu_part_capacity(),
+                                              ctx->own_fft ? 2 * spec_blocks(*ctx, 5) : 0));
         // static per-quantity fixed-point scales: the per-contribution bound maps
         // to 2^48, leaving 2^14 bound-sized contributions of headroom per cell
         double wmax = w_uniform;
@@ -305,6 +309,10 @@ struct aw_sim {
             j_staggered = false;
         }
         moments_ready = false;
+        if (ctx->own_fft) {
+            solve_fields_own(t);
+            return;
+        }
         // per run: rho, J -> src[0..3] and the R2C input block [run][4]; amu ->
         // src[7..10] and [run][7] entries 3..6 (fftin holds the copies rocFFT
         // may overwrite: [R x 4 grids][R x 7 grids])
@@ -338,6 +346,64 @@ struct aw_sim {
         fe.sL = 5 * nc;
         fe.sT = 3 * nc;
         form_e(fe, g, rp, t, s, R);
+    }
+
+    // solve_fields_em from the moments on the library's own transforms: the
+    // conversions, the field combinations and the maxima of the dcu scale ride
+    // in the solves' launches
+    void solve_fields_own(double t) {
+        const hipStream_t s = stream;
+        const int64_t nc = ncell(*ctx);
+        const int R = runs;
+        SpecSrc in4;  // rho, J
+        in4.acc = acc8.get();
+        in4.acc_rs = 8 * nc;
+        in4.out = src.get();
+        in4.out_rs = 11 * nc;
+        in4.inv = inv.get();
+        in4.inv_rs = 11;
+        in4.base = rbase.get();
+        SpecDst out5;
+        out5.out = elb.get();
+        out5.out1 = elb.get() + nc;
+        out5.out_rs = 5 * nc;
+        out5.form = SpecDst::kFormEl;
+        out5.e = ed3.get();
+        out5.e_rs = 3 * nc;
+        out5.pump = pump_args(g, rp, t);
+        out5.part = fmax_part.get();
+        spec_solve_elb(*ctx, in4, out5, rp.eps0, rp.c, rp.B0, j_staggered, R, s);
+        if (sort_requested || (cfg.sort_every > 0 && steps_since_sort >= cfg.sort_every)) do_sort();
+        dcu_scale_parts(fmax_part.get(), spec_blocks(*ctx, 5), dcu_abs, dcu_signed, umax,
+                        nullptr, cdcu.get(), inv.get() + 8, s, R, 11);
+        const float* Fd[6];
+        fields6(ed3.get(), Fd);
+        em_dcu(*ctx, particles(), tile_off.get(), nullptr, Fd, acc3.get(), cdcu.get(), bpt_dcu,
+               strays.get(), s, batch(3 * nc));
+        SpecSrc in7;  // dcu, then amu
+        in7.acc = acc3.get();
+        in7.acc_rs = 3 * nc;
+        in7.acc2 = acc8.get() + 4 * nc;
+        in7.acc2_rs = 8 * nc;
+        in7.split = 3;
+        in7.out = src.get();
+        in7.out_rs = 11 * nc;
+        in7.out_a = in7.out_b = 4;
+        in7.inv = inv.get();
+        in7.inv_rs = 11;
+        in7.inv_a = 8;
+        in7.inv_b = 1;
+        SpecDst out3;
+        out3.out = et.get();
+        out3.out1 = et.get() + nc;
+        out3.out_rs = 3 * nc;
+        out3.form = SpecDst::kFormEt;
+        out3.e = e3.get();
+        out3.e_rs = 3 * nc;
+        out3.el = elb.get();
+        out3.el_rs = 5 * nc;
+        out3.pump = out5.pump;
+        spec_solve_et(*ctx, in7, out3, rp.eps0, rp.c, rp.n0, R, s);
     }
 
     // darwin_fields + boris_em + migrate (include/pic/simulation.hpp:80-84)
@@ -622,8 +688,7 @@ struct aw_sim {
         }
         ctx->acc.zero(s);
         deposit_rho_fixed(*ctx, particles(), rp.qm, AW_DEPOSIT_BINNED, tile_off.get(), s);
-        fix_to_float(*ctx, rho.get(), true, s);
-        solve_es_contig(*ctx, ctx->rin.get(), E.get(), rp.eps0, s);
+        convert_solve_es(*ctx, ctx->acc.get(), rho.get(), E.get(), rp.eps0, nullptr, s);
         push_es(*ctx, particles(), Ex(), Ey(), rp, cfg.has_b0 != 0, true, s);
         strays.zero(s);  // afterwards cleared by each step's rho conversion
         fields_ready = true;
@@ -768,8 +833,7 @@ struct aw_sim {
             return;
         }
         if (!fields_ready) {
-            fix_to_float(*ctx, rho.get(), true, s, strays.get());
-            solve_es_contig(*ctx, ctx->rin.get(), E.get(), rp.eps0, s);
+            convert_solve_es(*ctx, ctx->acc.get(), rho.get(), E.get(), rp.eps0, strays.get(), s);
         }
         fields_ready = false;
         if (sort_requested || (cfg.sort_every > 0 && steps_since_sort >= cfg.sort_every)) do_sort();

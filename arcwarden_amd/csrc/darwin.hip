@@ -542,18 +542,6 @@ __global__ void convert_multi_kernel(unsigned long long* __restrict__ acc, float
     }
 }
 
-__device__ __forceinline__ double pump_ramp(double t, double trmp, double toff) {
-    if (t >= toff) return 0.0;
-    if (t < trmp) return t / trmp;
-    if (t > toff - trmp) return (toff - t) / trmp;
-    return 1.0;
-}
-
-struct PumpArgs {
-    int on;
-    double ex, ey, ez, k0, w0, trmp, toff, t, dx;
-};
-
 // E = (E_L + s*E_T) + pump(t) (combine_etotal_kernel, solver_darwin.hpp:134-144;
 // add_pump_kernel, pump.hpp:34-47); ET[0] may be null (s = 0).
 __global__ void form_e_kernel(FormE f, int nx, int ncell, PumpArgs p) {
@@ -574,13 +562,11 @@ __global__ void form_e_kernel(FormE f, int nx, int ncell, PumpArgs p) {
         ez = 1.0f * f.ET[2][c];
     }
     if (p.on && p.t < p.toff) {
-        const double x = (c % nx) * p.dx;
-        const double th = p.k0 * x - p.w0 * p.t;
-        const double r = pump_ramp(p.t, p.trmp, p.toff);
-        const double ct = cos(th), st = sin(th);
-        ex += (float)(p.ex * ct * r);
-        ey += (float)(-p.ey * st * r);
-        ez += (float)(p.ez * ct * r);
+        float px, py, pz;
+        dev::pump_at(p, c % nx, px, py, pz);
+        ex += px;
+        ey += py;
+        ez += pz;
     }
     f.E[0][c] = ex;
     f.E[1][c] = ey;
@@ -628,26 +614,28 @@ field_max_kernel(Field6 F, int ncell, float* __restrict__ part, long long sE, lo
 // dcu scale: per-contribution bound = |qm^2 w/area| (max|E| + umax max|B|);
 // S = 48 - ceil(log2(bound)) maps the bound to 2^48.  Writes the float
 // coefficient used by dcu_kernel and the inverse scale used by conversion.
-// dev (optional, device): {coef_abs, umax} measured from the particles.
-// Batched: one thread per run (threadIdx.x), run r reads part + 2*nb*r and
+// meas (optional, device): {coef_abs, umax} measured from the particles.
+// Batched: a workgroup per run (blockIdx.x), run r reads part + 2*nb*r and
 // writes c_dcu[r], inv_dcu + si*r.
-__global__ void dcu_scale_kernel(const float* __restrict__ part, int nb, double coef_abs,
-                                 double coef_signed, double umax, const double* __restrict__ dev,
-                                 float* __restrict__ c_dcu, double* __restrict__ inv_dcu, int runs,
-                                 int si) {
-    const int r = threadIdx.x;
-    if (r >= runs || blockIdx.x != 0) return;
+constexpr int kScaleWaves = 256;
+__global__ void __launch_bounds__(kScaleWaves)
+dcu_scale_kernel(const float* __restrict__ part, int nb, double coef_abs, double coef_signed,
+                 double umax, const double* __restrict__ meas, float* __restrict__ c_dcu,
+                 double* __restrict__ inv_dcu, int si) {
+    const int r = blockIdx.x;
     part += (size_t)2 * nb * r;
     c_dcu += r;
     inv_dcu += (size_t)si * r;
-    if (dev) {
-        coef_abs = dev[0];
-        umax = dev[1];
-    }
     float me = 0.f, mb = 0.f;
-    for (int i = 0; i < nb; ++i) {
+    for (int i = threadIdx.x; i < nb; i += kScaleWaves) {
         me = fmaxf(me, part[2 * i]);
         mb = fmaxf(mb, part[2 * i + 1]);
+    }
+    dev::block_max2(me, mb);
+    if (threadIdx.x != 0) return;
+    if (meas) {
+        coef_abs = meas[0];
+        umax = meas[1];
     }
     double bound = coef_abs * ((double)me + umax * (double)mb);
     if (!(bound > 1e-300)) bound = 1e-300;
@@ -875,9 +863,7 @@ void convert_multi(unsigned long long* acc, float* out, float* out2, int64_t nce
     AW_LAUNCH_CHECK();
 }
 
-// Batched (runs > 1): f carries run 0's pointers and the per-run strides.
-void form_e(const FormE& f, const aw_grid& g, const aw_run_params& rp, double t, hipStream_t s,
-            int runs) {
+PumpArgs pump_args(const aw_grid& g, const aw_run_params& rp, double t) {
     PumpArgs p{};
     p.on = rp.pump ? 1 : 0;
     p.ex = rp.pump_ex;
@@ -889,10 +875,21 @@ void form_e(const FormE& f, const aw_grid& g, const aw_run_params& rp, double t,
     p.toff = rp.pump_toff;
     p.t = t;
     p.dx = g.dx;
+    return p;
+}
+
+// Batched (runs > 1): f carries run 0's pointers and the per-run strides.
+void form_e(const FormE& f, const aw_grid& g, const aw_run_params& rp, double t, hipStream_t s,
+            int runs) {
+    const PumpArgs p = pump_args(g, rp, t);
     const int64_t nc = (int64_t)g.nx * g.ny;
     form_e_kernel<<<dim3(blocks_for(nc), runs), kThreads, 0, s>>>(f, g.nx, (int)nc, p);
     AW_LAUNCH_CHECK();
 }
+
+void dcu_scale_parts(const float* part, int nb, double coef_abs, double coef_signed, double umax,
+                     const double* dev, float* c_dcu, double* inv_dcu, hipStream_t s, int runs,
+                     int si);
 
 // Batched (runs > 1): F holds run 0's fields, E components at stride sE and
 // B at stride sB per run; part holds dcu_part_capacity(ncell) floats per run,
@@ -905,8 +902,15 @@ void dcu_scale(const float* const* F, int64_t ncell, float* part, double coef_ab
     Field6 f6{{F[0], F[1], F[2], F[3], F[4], F[5]}};
     field_max_kernel<<<dim3(nb, runs), kThreads, 0, s>>>(f6, (int)ncell, part, sE, sB);
     AW_LAUNCH_CHECK();
-    dcu_scale_kernel<<<1, 64, 0, s>>>(part, nb, coef_abs, coef_signed, umax, dev, c_dcu, inv_dcu,
-                                      runs, si);
+    dcu_scale_parts(part, nb, coef_abs, coef_signed, umax, dev, c_dcu, inv_dcu, s, runs, si);
+}
+
+// the same from maxima already taken, nb pairs per run
+void dcu_scale_parts(const float* part, int nb, double coef_abs, double coef_signed, double umax,
+                     const double* dev, float* c_dcu, double* inv_dcu, hipStream_t s, int runs,
+                     int si) {
+    dcu_scale_kernel<<<runs, kScaleWaves, 0, s>>>(part, nb, coef_abs, coef_signed, umax, dev, c_dcu,
+                                                  inv_dcu, si);
     AW_LAUNCH_CHECK();
 }
 

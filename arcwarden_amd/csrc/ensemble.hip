@@ -262,7 +262,11 @@ struct aw_ensemble {
 
     void convert_and_solve() {
         // rho^n for every run; rin receives the R2C input copy, strays reset
-        fix_to_float_add(acc.get(), rho.get(), nctot, fix_log2, true, stream, true, strays.get(),
+        // (on the library's own transforms each size's solve converts for itself)
+        const bool own = std::all_of(groups.begin(), groups.end(), [&](const Group& gr) {
+            return runs[gr.first].ctx->own_fft;
+        });
+        if (!own) fix_to_float_add(acc.get(), rho.get(), nctot, fix_log2, true, stream, true, strays.get(),
                          rin.get(), (int)runs.size(), rbase.get());
         // one batched solve per grid size; the sizes touch disjoint buffers
         // (each its own plans, work area and k-space scratch), so they fork
@@ -276,8 +280,30 @@ struct aw_ensemble {
         for (size_t g = 0; g < groups.size(); ++g) {
             const Group& gr = groups[g];
             const size_t lane = nside ? g % (nside + 1) : 0;
-            solve_es_batch(*runs[gr.first].ctx, gr.count, rin.get() + gr.cbase,
-                           E.get() + 2 * gr.cbase, eps0, lane ? side[lane - 1] : stream);
+            aw_ctx& c = *runs[gr.first].ctx;
+            const hipStream_t sg = lane ? side[lane - 1] : stream;
+            if (!own) {
+                solve_es_batch(c, gr.count, rin.get() + gr.cbase, E.get() + 2 * gr.cbase, eps0, sg);
+                continue;
+            }
+            const int64_t nc = ncell(c);
+            SpecSrc in;
+            in.acc = acc.get() + gr.cbase;
+            in.acc_rs = nc;
+            in.out = rho.get() + gr.cbase;
+            in.out_rs = nc;
+            in.inv0 = std::ldexp(1.0, -fix_log2);
+            in.base = rbase.get() + gr.cbase;
+            in.base_cell = 1;
+            if (g == 0) {
+                in.counter = strays.get();
+                in.ncounter = (int)runs.size();
+            }
+            SpecDst out;
+            out.out = E.get() + 2 * gr.cbase;
+            out.out1 = out.out + nc;
+            out.out_rs = 2 * nc;
+            spec_solve_es(c, in, out, eps0, gr.count, sg);
         }
         for (size_t i = 0; i < nside; ++i) {
             AW_HIP(hipEventRecord(fork_join[1 + i], side[i]));

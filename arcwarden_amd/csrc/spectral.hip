@@ -1,4 +1,7 @@
-// spectral.hip -- rocFFT plans and the pointwise k-space solves.
+// spectral.hip -- rocFFT plans and the pointwise k-space solves, for the grids
+// whose sides the library's own transforms (fft.hip) do not take: a prime
+// factor above 61, lines too long for LDS, or large powers of two.  The entry
+// points below choose.
 //
 // Reference: CufftPlan2D (include/pic/fft.hpp:26-93), SpectralEngine
 // (include/pic/spectral.hpp:106-149), es_poisson_field_kernel
@@ -8,6 +11,8 @@
 // (the reference runs scale_inplace_kernel after every C2R, spectral.hpp:97-101).
 #include "aw_internal.hpp"
 
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 
 namespace aw {
@@ -92,14 +97,17 @@ rocfft_plan make_plan(const aw_ctx& c, bool forward, int batch, double scale) {
 void init_fft(aw_ctx& c) {
     std::call_once(g_rocfft_once, [] { rocfft_setup(); });
     const double inv = 1.0 / ((double)c.g.nx * (double)c.g.ny);
-    c.r2c = make_plan(c, true, 1, 1.0);
+    init_own_fft(c);
+    c.r2c = make_plan(c, true, 1, 1.0);  // aw_fft_r2c, aw_fft_c2r
     c.c2r = make_plan(c, false, 1, inv);
-    c.c2r2 = make_plan(c, false, 2, inv);
-    c.r2c2 = make_plan(c, true, 2, 1.0);
-    c.r2c3 = make_plan(c, true, 3, 1.0);
-    c.c2r3 = make_plan(c, false, 3, inv);
+    if (!c.own_fft) {
+        c.c2r2 = make_plan(c, false, 2, inv);
+        c.r2c2 = make_plan(c, true, 2, 1.0);
+        c.c2r3 = make_plan(c, false, 3, inv);
+    }
     size_t work = 0;
-    for (rocfft_plan p : {c.r2c, c.c2r, c.c2r2, c.r2c2, c.r2c3, c.c2r3}) {
+    for (rocfft_plan p : {c.r2c, c.c2r, c.c2r2, c.r2c2, c.c2r3}) {
+        if (!p) continue;
         size_t w = 0;
         AW_FFT(rocfft_plan_get_work_buffer_size(p, &w));
         work = std::max(work, w);
@@ -111,7 +119,7 @@ void init_fft(aw_ctx& c) {
 // Darwin batches: R2C x4 [rho|Jx|Jy|Jz], R2C x7 [dcu(3)|amu(4)], C2R x5
 // [ELx|ELy|Bx|By|Bz] (C2R x3 [ETx|ETy|ETz] is shared with the base set).
 void enable_em_fft(aw_ctx& c) {
-    if (c.r2c4) return;
+    if (c.own_fft || c.r2c4) return;
     const double inv = 1.0 / ((double)c.g.nx * (double)c.g.ny);
     c.r2c4 = make_plan(c, true, 4, 1.0);
     c.r2c7 = make_plan(c, true, 7, 1.0);
@@ -129,6 +137,10 @@ void enable_em_fft(aw_ctx& c) {
 void enable_em_batch_fft(aw_ctx& c, int R) {
     if (c.em_batch == R) return;
     AW_REQUIRE(c.em_batch == 0, "Darwin batch plans already prepared for another size");
+    if (c.own_fft) {
+        c.em_batch = R;
+        return;
+    }
     enable_em_fft(c);
     const double inv = 1.0 / ((double)c.g.nx * (double)c.g.ny);
     c.r2c4B = make_plan(c, true, 4 * R, 1.0);
@@ -146,7 +158,7 @@ void enable_em_batch_fft(aw_ctx& c, int R) {
 }
 
 void destroy_fft(aw_ctx& c) noexcept {
-    for (rocfft_plan* p : {&c.r2c, &c.c2r, &c.c2r2, &c.r2c2, &c.r2c3, &c.c2r3, &c.r2c4, &c.r2c7,
+    for (rocfft_plan* p : {&c.r2c, &c.c2r, &c.c2r2, &c.r2c2, &c.c2r3, &c.r2c4, &c.r2c7,
                            &c.c2r5, &c.r2cB, &c.c2rB, &c.r2c4B, &c.c2r5B, &c.r2c7B, &c.c2r3B})
         if (*p) {
             rocfft_plan_destroy(*p);
@@ -165,6 +177,57 @@ void fft_exec(aw_ctx& c, rocfft_plan plan, void* in, void* out, hipStream_t s) {
     void* ib[1] = {in};
     void* ob[1] = {out};
     AW_FFT(rocfft_execute(plan, ib, ob, c.info));
+}
+
+namespace {
+// runs of FP32 rho -> (Ex, Ey), rs apart, on the library's own transforms
+void own_es(aw_ctx& c, const float* rho, float* Ex, float* Ey, int64_t rs, double eps0, int runs,
+            hipStream_t s) {
+    SpecSrc in;
+    in.in = rho;
+    in.in_rs = ncell(c);
+    SpecDst out;
+    out.out = Ex;
+    out.out1 = Ey;
+    out.out_rs = rs;
+    spec_solve_es(c, in, out, eps0, runs, s);
+}
+
+// nin contiguous FP32 grids a run in, nout out
+std::pair<SpecSrc, SpecDst> own_grids(aw_ctx& c, const float* src, int nin, float* dst, int nout) {
+    const int64_t nc = ncell(c);
+    SpecSrc in;
+    in.in = src;
+    in.in_rs = nin * nc;
+    SpecDst out;
+    out.out = dst;
+    out.out1 = dst + nc;
+    out.out_rs = nout * nc;
+    return {in, out};
+}
+}  // namespace
+
+void convert_solve_es(aw_ctx& c, unsigned long long* acc, float* rho, float* E2, double eps0,
+                      unsigned long long* counter, hipStream_t s) {
+    const int64_t nc = ncell(c);
+    if (!c.own_fft) {
+        c.rin.reserve((size_t)nc);
+        fix_to_float_add(acc, rho, nc, c.fix_log2, true, s, true, counter, c.rin.get(), 1, nullptr,
+                         c.rho_base);
+        solve_es_contig(c, c.rin.get(), E2, eps0, s);
+        return;
+    }
+    SpecSrc in;
+    in.acc = acc;
+    in.out = rho;
+    in.inv0 = std::ldexp(1.0, -c.fix_log2);
+    in.base_val = c.rho_base;
+    in.counter = counter;
+    in.ncounter = counter ? 1 : 0;
+    SpecDst out;
+    out.out = E2;
+    out.out1 = E2 + nc;
+    spec_solve_es(c, in, out, eps0, 1, s);
 }
 
 // rho -> (Ex, Ey) with E2 = [Ex | Ey] contiguous (2*nx*ny floats): one R2C,
@@ -211,6 +274,10 @@ __global__ void es_kspace_batch_kernel(const float2* __restrict__ rk, float2* __
 
 void enable_batch_fft(aw_ctx& c, int batch) {
     if (c.fft_batch == batch) return;
+    if (c.own_fft) {
+        c.fft_batch = batch;
+        return;
+    }
     for (rocfft_plan* p : {&c.r2cB, &c.c2rB})
         if (*p) {
             rocfft_plan_destroy(*p);
@@ -233,6 +300,10 @@ void enable_batch_fft(aw_ctx& c, int batch) {
 void solve_es_batch(aw_ctx& c, int batch, float* rho_in, float* E2B, double eps0,
                     hipStream_t s) {
     AW_REQUIRE(c.fft_batch == batch, "batched plans not prepared for this batch");
+    if (c.own_fft) {
+        own_es(c, rho_in, E2B, E2B + ncell(c), 2 * ncell(c), eps0, batch, s);
+        return;
+    }
     const int64_t nk = nkmodes(c);
     c.ktmp.reserve((size_t)6 * nk * batch);
     float2* rk = reinterpret_cast<float2*>(c.ktmp.get());
@@ -246,6 +317,10 @@ void solve_es_batch(aw_ctx& c, int batch, float* rho_in, float* E2B, double eps0
 }
 
 void solve_es_contig(aw_ctx& c, const float* rho, float* E2, double eps0, hipStream_t s) {
+    if (c.own_fft) {
+        own_es(c, rho, E2, E2 + ncell(c), 0, eps0, 1, s);
+        return;
+    }
     const int64_t nk = nkmodes(c);
     c.ktmp.reserve((size_t)6 * nk);
     float2* rk = reinterpret_cast<float2*>(c.ktmp.get());
@@ -373,6 +448,11 @@ __global__ void darwin_et_kernel(const float2* __restrict__ src, float2* __restr
 void solve_darwin_elb(aw_ctx& c, const float* src4, float* out5, double eps0, double cl,
                       const float B0[3], hipStream_t s, bool stag, int runs) {
     AW_REQUIRE(runs == 1 || runs == c.em_batch, "Darwin batch plans not prepared");
+    if (c.own_fft) {
+        const auto [in, out] = own_grids(c, src4, 4, out5, 5);
+        spec_solve_elb(c, in, out, eps0, cl, B0, stag, runs, s);
+        return;
+    }
     const int64_t nk = nkmodes(c);
     c.ktmp.reserve((size_t)2 * 12 * nk * runs);
     float2* k4 = reinterpret_cast<float2*>(c.ktmp.get());
@@ -390,6 +470,11 @@ void solve_darwin_elb(aw_ctx& c, const float* src4, float* out5, double eps0, do
 void solve_darwin_et(aw_ctx& c, const float* src7, float* out3, double eps0, double cl,
                      double n0, hipStream_t s, int runs) {
     AW_REQUIRE(runs == 1 || runs == c.em_batch, "Darwin batch plans not prepared");
+    if (c.own_fft) {
+        const auto [in, out] = own_grids(c, src7, 7, out3, 3);
+        spec_solve_et(c, in, out, eps0, cl, n0, runs, s);
+        return;
+    }
     const int64_t nk = nkmodes(c);
     c.ktmp.reserve((size_t)2 * 12 * nk * runs);
     float2* k7 = reinterpret_cast<float2*>(c.ktmp.get());
@@ -404,6 +489,10 @@ void solve_darwin_et(aw_ctx& c, const float* src7, float* out3, double eps0, dou
 
 // General form with separate output buffers.
 void solve_es(aw_ctx& c, const float* rho, float* Ex, float* Ey, double eps0, hipStream_t s) {
+    if (c.own_fft) {
+        own_es(c, rho, Ex, Ey, 0, eps0, 1, s);
+        return;
+    }
     const int64_t nk = nkmodes(c);
     c.ktmp.reserve((size_t)6 * nk);
     float2* rk = reinterpret_cast<float2*>(c.ktmp.get());
