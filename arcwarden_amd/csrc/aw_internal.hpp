@@ -282,6 +282,7 @@ struct EskExtra {
     // (unused, max |uz|) with w_uniform
     bool fixed = false;
     int fixed_per_w = 0;
+    bool cleared = false;  // c.jacc cleared and c.jbound set by the caller (fixed)
     float fixed_bound[2] = {0.f, 0.f};
     const int32_t* slice_off = nullptr;
     float *xw = nullptr, *yw = nullptr;

@@ -449,6 +449,7 @@ EskArgs setup(aw_ctx& c, const float* x0, const float* y0, const aw_particles& p
         AW_REQUIRE(ex.fixed_bound[0] >= 0.f && ex.fixed_bound[1] >= 0.f &&
                        std::isfinite(ex.fixed_bound[0]) && std::isfinite(ex.fixed_bound[1]),
                    "the current's fixed scale bounds must be finite and non-negative");
+        if (ex.cleared) return a;
         const int nb = (int)std::min<int64_t>((3 * nc + kThreads - 1) / kThreads,
                                               8 * std::max(1, c.num_cu));
         esk_begin_kernel<<<nb, kThreads, 0, s>>>(c.jacc.get(), 3 * nc, ex.fixed_bound[0],

@@ -87,13 +87,21 @@ __device__ __forceinline__ void ampere_cell(const Mesh& m, int c) {
     m.ez[c] = m.ez[c] + m.dt * (m.c2 * (dby_x - dbx_y) - m.jz[c]);
 }
 
-// Faraday half step (include/pic/yee2d.hpp:70-81); zero_j also clears the
-// current for the step's deposit
-__global__ void __launch_bounds__(kThreads) faraday_kernel(Mesh m, float h, int zero_j) {
+// Faraday half step (include/pic/yee2d.hpp:70-81).  For the step's current it
+// also clears the accumulators (acc, three grids) and sets its fixed bounds.
+__global__ void __launch_bounds__(kThreads)
+faraday_kernel(Mesh m, float h, unsigned long long* __restrict__ acc, float2 bound,
+               unsigned int* __restrict__ bounds) {
     const int c = blockIdx.x * kThreads + threadIdx.x;
-    if (c >= m.nx * m.ny) return;
+    const int64_t nc = (int64_t)m.nx * m.ny;
+    if (c >= nc) return;
     faraday_cell(m, h, c);
-    if (zero_j) m.jx[c] = m.jy[c] = m.jz[c] = 0.f;
+    if (!acc) return;
+    acc[c] = acc[nc + c] = acc[2 * nc + c] = 0ull;
+    if (c == 0) {
+        bounds[0] = __float_as_uint(bound.x);
+        bounds[1] = __float_as_uint(bound.y);
+    }
 }
 
 // Ampere step (include/pic/yee2d.hpp:84-97)
@@ -656,6 +664,101 @@ yee_push_esk_tiles_kernel(PushArgs a, Mesh m, aw_run_params rp, PushTiles t, esk
     }
 }
 
+// One-row grids whose current fits LDS: a workgroup per CU keeps the whole
+// line's current there and pushes its share of the particles, the fields from
+// the mesh, in one pass over them (52 B a delta-f particle; the push and the
+// deposit by themselves move 100).  Particles in any order.  Where they still
+// lie cell by cell, every move of a wavefront adds to the same words: the
+// wavefront then sums its quanta across the lanes and one lane adds them.
+// 3.4 M delta-f particles on 5000 cells: push 66 us + deposit 46 us before,
+// 93 us.
+constexpr int kRowThreads = 1024;
+
+template <bool PLAIN, bool NOPR>
+__global__ void __launch_bounds__(kRowThreads)
+yee_push_esk_row_kernel(PushArgs a, Mesh m, aw_run_params rp, esk::EskArgs e, int qslots,
+                        unsigned long long* __restrict__ acc) {
+    extern __shared__ unsigned long long s_mem[];
+    const int nc = m.nx;
+    MoveQueue queue{reinterpret_cast<float*>(s_mem + 3 * nc) +
+                        (threadIdx.x >> 6) * qslots * MoveQueue::kFloats,
+                    qslots};
+    for (int c = threadIdx.x; c < 3 * nc; c += kRowThreads) s_mem[c] = 0ull;
+    __syncthreads();
+    const MeshGather gat{m};
+    double kc[3];
+    esk::esk_coefs(e, kc);
+    auto general = [&](float x0, float y0, float x1, float y1, float uz, float w) {
+        esk::EskMove mv;
+        esk::esk_prepare_v(e, x0, y0, x1, y1, uz, e.per_w ? (double)w : e.w_uniform, kc, mv);
+        int gx[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) gx[k] = dev::wrapfar(mv.sh.ib + k, nc);
+        esk::esk_emit<true>(mv, [&](int q, int k, int, unsigned long long v) {
+            atomicAdd(&s_mem[q * nc + gx[k - 1]], v);
+        });
+    };
+    const int64_t stride = (int64_t)kRowThreads * gridDim.x;
+    for (int64_t base = (int64_t)blockIdx.x * kRowThreads; base < a.n; base += stride) {
+        const int64_t t = base + threadIdx.x;
+        bool leaves = false;
+        int cell = -1;
+        PushOut o;
+        unsigned long long col[5] = {};  // Jx at the cell, Jy and Jz at it and the next
+        if (t < a.n) {
+            push_one<PLAIN, MeshGather, NOPR>(a, m, rp, (int)t, load_particle(a, (int)t), o, gat);
+            a.x[t] = dev::wrap_coord(o.x1, (float)m.nx);
+            a.y[t] = dev::wrap_coord(o.y1, (float)m.ny);
+            a.ux[t] = o.vx;
+            a.uy[t] = o.vy;
+            a.uz[t] = o.vz;
+            const float flx = floorf(o.x0), fly = floorf(o.y0);
+            leaves = !(flx < (float)nc &&
+                       dev::esk_same_cell(o.x0, o.y0, o.x1, o.y1, flx, fly, m.nx, 1));
+            if (!leaves) {
+                cell = (int)flx;
+                const dev::EskCell c =
+                    dev::esk_cell((double)(o.x0 - flx), (double)(o.y0 - fly),
+                                  (double)(o.x1 - flx), (double)(o.y1 - fly));
+                const double qw = e.qm * (e.per_w ? (double)o.w : e.w_uniform);
+                esk::esk_emit_cell<true>(
+                    c, dev::clamp_fix_f64(-qw * kc[0]), dev::clamp_fix_f64(-qw * kc[1]),
+                    dev::clamp_fix_f64(qw * (double)o.uz * kc[2] * (16.0 / 12.0)),
+                    [&](int q, int k, int, unsigned long long v) {
+                        col[q == 0 ? 0 : 2 * q - 1 + (k - 1)] = v;
+                    });
+            }
+        }
+        const unsigned long long in = __ballot(cell >= 0);
+        if (in) {
+            const int lead = __ffsll((long long)in) - 1;
+            const int c0 = __shfl(cell, lead, 64);
+            const bool uniform = __ballot(cell >= 0 && cell != c0) == 0ull;
+            if (uniform) {
+#pragma unroll
+                for (int k = 0; k < 5; ++k)
+#pragma unroll
+                    for (int d = 32; d > 0; d >>= 1) col[k] += __shfl_xor(col[k], d, 64);
+            }
+            if (uniform ? (int)(threadIdx.x & 63) == lead : cell >= 0) {
+                const int next = cell + 1 == nc ? 0 : cell + 1;
+                atomicAdd(&s_mem[cell], col[0]);
+                atomicAdd(&s_mem[nc + cell], col[1]);
+                atomicAdd(&s_mem[nc + next], col[2]);
+                atomicAdd(&s_mem[2 * nc + cell], col[3]);
+                atomicAdd(&s_mem[2 * nc + next], col[4]);
+            }
+        }
+        queue.push(leaves, o.x0, o.y0, o.x1, o.y1, o.uz, o.w, general);
+    }
+    queue.drain(general);
+    __syncthreads();
+    for (int c = threadIdx.x; c < 3 * nc; c += kRowThreads) {
+        const unsigned long long v = s_mem[c];
+        if (v) atomicAdd(&acc[c], v);
+    }
+}
+
 // per-workgroup max |a[i]|
 __global__ void __launch_bounds__(kThreads) max_abs_kernel(const float* __restrict__ a, int64_t n,
                                                            float* __restrict__ part) {
@@ -700,28 +803,57 @@ binomial_kernel(const float* __restrict__ src, float* __restrict__ dst, Mesh m) 
     dst[blockIdx.y * nc + c] = binomial_at(src + blockIdx.y * nc, m, c);
 }
 
-// the current's conversion (J += acc 2^-S) and every smoothing pass of
-// component blockIdx.x in LDS, for grids of up to kSmoothLdsCells
-__global__ void __launch_bounds__(1024)
+// The current of the accumulators and every smoothing pass, a workgroup per
+// tile and component: the tile and `passes` cells around it are converted into
+// LDS and shrink by one cell a pass, so the passes need no launch, and no
+// grid, between them.  5000x1, 3 passes: 14.4 us with a
+// workgroup a component, 4.8 us so; 625x625, 3 passes: 25 us in four launches,
+// 18 us.  One row (ny = 1) is 256 cells wide, its three aliased rows the same
+// one.
+constexpr int kSmoothTile = 256;   // cells: 32 x 8, or 256 x 1
+constexpr int kMaxFusedPasses = 4;
+
+template <bool ONE_ROW>
+__global__ void __launch_bounds__(kSmoothTile)
 convert_smooth_kernel(float* __restrict__ j, Mesh m, int passes,
                       const unsigned long long* __restrict__ acc, esk::EskArgs e) {
-    extern __shared__ float s_c[];
-    const int nc = m.nx * m.ny, q = blockIdx.x;
+    constexpr int TX = ONE_ROW ? 256 : 32, TY = ONE_ROW ? 1 : 8;
+    constexpr int MW = TX + 2 * kMaxFusedPasses, MH = ONE_ROW ? 1 : TY + 2 * kMaxFusedPasses;
+    __shared__ float s_a[MW * MH], s_b[MW * MH];
+    const int q = blockIdx.z, x0 = blockIdx.x * TX - passes, y0 = ONE_ROW ? 0 : blockIdx.y * TY - passes;
+    const int W = TX + 2 * passes, H = ONE_ROW ? 1 : TY + 2 * passes;
+    const int64_t nc = (int64_t)m.nx * m.ny;
     int S[3];
     esk::esk_exponents(e, S);
-    float* g = j + (int64_t)q * nc;
-    float *cur = s_c, *nxt = s_c + nc;
-    for (int c = threadIdx.x; c < nc; c += blockDim.x)
-        cur[c] = g[c] + esk::esk_value((long long)acc[(int64_t)q * nc + c], S[q]);
+    for (int t = threadIdx.x; t < W * H; t += kSmoothTile) {
+        const int r = t / W, c = t - r * W;
+        const int64_t g = (int64_t)dev::wrapfar(y0 + r, m.ny) * m.nx + dev::wrapfar(x0 + c, m.nx);
+        s_a[t] = 0.f + esk::esk_value((long long)acc[q * nc + g], S[q]);
+    }
     __syncthreads();
-    for (int k = 0; k < passes; ++k) {
-        for (int c = threadIdx.x; c < nc; c += blockDim.x) nxt[c] = binomial_at(cur, m, c);
+    float *cur = s_a, *nxt = s_b;
+    for (int k = 1; k <= passes; ++k) {
+        const int w = W - 2 * k, h = ONE_ROW ? 1 : H - 2 * k;
+        for (int t = threadIdx.x; t < w * h; t += kSmoothTile) {
+            const int r = t / w, at = (ONE_ROW ? 0 : (r + k) * W) + t - r * w + k;
+            const float wt[3] = {0.25f, 0.5f, 0.25f};
+            float sum = 0.f;
+#pragma unroll
+            for (int dj = -1; dj <= 1; ++dj)
+#pragma unroll
+                for (int di = -1; di <= 1; ++di)
+                    sum = fmaf(wt[di + 1] * wt[dj + 1], cur[at + (ONE_ROW ? 0 : dj * W) + di], sum);
+            nxt[at] = sum;
+        }
         __syncthreads();
         float* t = cur;
         cur = nxt;
         nxt = t;
     }
-    for (int c = threadIdx.x; c < nc; c += blockDim.x) g[c] = cur[c];
+    const int c = threadIdx.x % TX, r = threadIdx.x / TX;
+    const int gx = blockIdx.x * TX + c, gy = ONE_ROW ? 0 : blockIdx.y * TY + r;
+    if (gx < m.nx && gy < m.ny)
+        j[q * nc + (int64_t)gy * m.nx + gx] = cur[(ONE_ROW ? 0 : (r + passes) * W) + c + passes];
 }
 
 // every pass of grid blockIdx.x in LDS, for grids of up to kSmoothLdsCells
@@ -1123,8 +1255,7 @@ struct aw_maxwell {
     }
 
     // rp.jfilter binomial passes, in place, over ncomp consecutive grids
-    void smooth(float* a, int ncomp) {
-        const int J = rp.jfilter;
+    void smooth(float* a, int ncomp, int J) {
         if (J <= 0) return;
         const Mesh m = mesh();
         const int64_t n = nc();
@@ -1190,20 +1321,21 @@ struct aw_maxwell {
         }
     }
 
-    // J += the accumulated current, then rp.jfilter smoothing passes: one LDS
-    // launch for the three components of a small grid
+    // J = the accumulated current after rp.jfilter smoothing passes
     void convert_and_smooth(const esk::EskArgs& e) {
         const Mesh m = mesh();
-        const int64_t n = nc();
-        const size_t lds = (size_t)(2 * n) * sizeof(float);
-        if (rp.jfilter > 0 && n <= kSmoothLdsCells && lds <= ctx->lds_per_block) {
-            convert_smooth_kernel<<<3, kSmoothThreads, lds, stream>>>(m.jx, m, rp.jfilter,
-                                                                     ctx->jacc.get(), e);
-            AW_LAUNCH_CHECK();
-            return;
-        }
-        esk::convert(*ctx, e, m.jx, m.jy, m.jz, stream);
-        smooth(m.jx, 3);
+        const int fused = std::min(rp.jfilter, kMaxFusedPasses);
+        const bool one_row = g.ny == 1;
+        const int tx = one_row ? 256 : 32, ty = one_row ? 1 : 8;
+        const dim3 grid((g.nx + tx - 1) / tx, (g.ny + ty - 1) / ty, 3);
+        if (one_row)
+            convert_smooth_kernel<true><<<grid, kSmoothTile, 0, stream>>>(m.jx, m, fused,
+                                                                          ctx->jacc.get(), e);
+        else
+            convert_smooth_kernel<false><<<grid, kSmoothTile, 0, stream>>>(m.jx, m, fused,
+                                                                           ctx->jacc.get(), e);
+        AW_LAUNCH_CHECK();
+        smooth(m.jx, 3, rp.jfilter - fused);
     }
 
     // Stable physical sort of the particles into tile order, in place in the
@@ -1257,15 +1389,38 @@ struct aw_maxwell {
         const Mesh m = mesh();
         const int nb = blocks_for(nc());
         const float h = 0.5f * (float)rp.dt;
-        // the first half step also clears J for the particles' current
-        faraday_kernel<<<nb, kThreads, 0, stream>>>(m, h, p.n > 0 ? 1 : 0);
-        AW_LAUNCH_CHECK();
+        // the first half step also clears the accumulators of the particles'
+        // current and sets its bounds
+        EskExtra ex;
+        float wm = 0.f;
+        const float ucap = (float)(2.0 * std::max(1.0, rp.c));
         if (p.n > 0) {
             AW_REQUIRE(!rp.deltaf || (df && df->wd), "delta-f run without a weight array");
             AW_REQUIRE(!rp.deltaf || rp.df_wprec != 1 || df->wc,
                        "df_wprec = 1 needs the compensation array");
             AW_REQUIRE(!rp.deltaf || rp.df_wprec != 2 || df->wdd,
                        "df_wprec = 2 needs the FP64 weight array");
+            // The current's fixed-point scale comes from bounds fixed before the
+            // push: |uz/gamma| <= 2 max(1, c) (below c for the relativistic
+            // push), |w| <= the run's largest weight, and |w wd| <= 8 |w|
+            // (wd is clamped to [-8, 1)).  Particles past them set the guard,
+            // which synchronize reports.
+            wm = weight_max(p);
+            ex.fixed = ex.cleared = true;
+            ex.fixed_per_w = rp.deltaf || p.w ? 1 : 0;
+            const float wb = rp.deltaf ? 8.f * wm : wm;
+            ex.fixed_bound[0] = ex.fixed_per_w ? wb : 0.f;
+            ex.fixed_bound[1] = ex.fixed_per_w
+                                    ? std::nextafter((float)((double)wb * ucap), INFINITY)
+                                    : ucap;
+            ctx->jacc.reserve((size_t)(3 * nc()));
+            ctx->jbound.reserve(2);
+        }
+        faraday_kernel<<<nb, kThreads, 0, stream>>>(
+            m, h, p.n > 0 ? ctx->jacc.get() : nullptr,
+            make_float2(ex.fixed_bound[0], ex.fixed_bound[1]), ctx->jbound.get());
+        AW_LAUNCH_CHECK();
+        if (p.n > 0) {
             const size_t n = (size_t)p.n;
             // the current's uz/gamma is taken before the walls damp u (bnd_x = 2)
             const bool own_vz = rp.rel || rp.bnd_x;
@@ -1280,7 +1435,13 @@ struct aw_maxwell {
                                   p.n >= 16 * ncl) &&
                                 (double)p.n / (double)ncl >= 8.0;
             const bool fused = rp.tile_sort > 0 || binned;
-            if (!fused) {
+            // one row whose current takes AUTO's whole-grid LDS policy: one pass
+            constexpr size_t kSlot =
+                (kRowThreads / 64) * MoveQueue::kFloats * sizeof(float);
+            const size_t row_lds = (size_t)(3 * ncl) * sizeof(unsigned long long);
+            const bool row = !fused && g.ny == 1 && p.n >= 16 * ncl &&
+                             row_lds + 8 * kSlot <= ctx->lds_per_block;
+            if (!fused && !row) {
                 x0.reserve(n);
                 y0.reserve(n);
                 if (own_vz) vz.reserve(n);
@@ -1297,31 +1458,18 @@ struct aw_maxwell {
             a.wd = rp.deltaf ? df->wd : nullptr;
             a.wc = rp.deltaf ? df->wc : nullptr;
             a.wdd = rp.deltaf ? df->wdd : nullptr;
-            a.x0 = fused ? nullptr : x0.get();
-            a.y0 = fused ? nullptr : y0.get();
-            a.vz = !fused && own_vz ? vz.get() : nullptr;
-            a.wdep = !fused && rp.deltaf ? wdep.get() : nullptr;
+            const bool apart = !fused && !row;  // the push and the current's deposit
+            a.x0 = apart ? x0.get() : nullptr;
+            a.y0 = apart ? y0.get() : nullptr;
+            a.vz = apart && own_vz ? vz.get() : nullptr;
+            a.wdep = apart && rp.deltaf ? wdep.get() : nullptr;
             a.n = (int)p.n;
             a.tnow = tnow;
             a.rdx = 1.0 / (double)m.dx;
             a.rdy = 1.0 / (double)m.dy;
-            // The current's fixed-point scale comes from bounds fixed before the
-            // push: |uz/gamma| <= 2 max(1, c) (below c for the relativistic
-            // push), |w| <= the run's largest weight, and |w wd| <= 8 |w|
-            // (wd is clamped to [-8, 1)).  Particles past them set the guard,
-            // which synchronize reports.
-            const float wm = weight_max(p);
-            a.ucap = (float)(2.0 * std::max(1.0, rp.c));
+            a.ucap = ucap;
             a.wmax = wm;
             a.guard = jguard.get();
-            EskExtra ex;
-            ex.fixed = true;
-            ex.fixed_per_w = rp.deltaf || p.w ? 1 : 0;
-            const float wb = rp.deltaf ? 8.f * wm : wm;
-            ex.fixed_bound[0] = ex.fixed_per_w ? wb : 0.f;
-            ex.fixed_bound[1] = ex.fixed_per_w
-                                    ? std::nextafter((float)((double)wb * a.ucap), INFINITY)
-                                    : a.ucap;
             if (fused) {
                 PushTiles t{};
                 if (binned) {
@@ -1368,6 +1516,22 @@ struct aw_maxwell {
                 hipLaunchKernelGGL(kern,
                                    dim3(ctx->ntiles * t.bpt), dim3(kThreads), sh, stream, a, m, rp,
                                    t, e, ctx->jacc.get());
+                AW_LAUNCH_CHECK();
+                convert_and_smooth(e);
+            } else if (row) {
+                const int slots = (int)std::min<size_t>(kQueueSlots,
+                                                        (ctx->lds_per_block - row_lds) / kSlot);
+                const esk::EskArgs e = esk::setup(*ctx, nullptr, nullptr, p, rp.qm, rp.dt, stream,
+                                                  ex);
+                const bool nopr = !(rp.pump || rp.rel);
+                auto kern = nopr && !(rp.b0_prof || rp.deltaf || rp.bnd_x)
+                                ? yee_push_esk_row_kernel<true, false>
+                            : nopr ? yee_push_esk_row_kernel<false, true>
+                                   : yee_push_esk_row_kernel<false, false>;
+                const int nb1 = (int)std::min<int64_t>((p.n + kRowThreads - 1) / kRowThreads,
+                                                       std::max(1, ctx->num_cu));
+                kern<<<nb1, kRowThreads, row_lds + slots * kSlot, stream>>>(a, m, rp, e, slots,
+                                                                           ctx->jacc.get());
                 AW_LAUNCH_CHECK();
                 convert_and_smooth(e);
             } else {
@@ -1445,7 +1609,7 @@ struct aw_maxwell {
         } else {
             zero(rho.get(), n);
         }
-        smooth(rho.get(), 1);
+        smooth(rho.get(), 1, rp.jfilter);
         gauss_kernel<<<blocks_for(n), kThreads, 0, stream>>>(mesh(), rho.get(), rres.get());
         AW_LAUNCH_CHECK();
         if (!have_ref) {
