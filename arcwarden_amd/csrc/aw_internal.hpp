@@ -207,6 +207,7 @@ struct SortScratch {
     DevBuf<uint32_t> table, sums;
     DevBuf<uint32_t> colsum;  // tile sort: per (chunk block, tile) sums, then tile bases
     DevBuf<int32_t> bin_off, bin_perm;  // tile bins of the last binned deposit
+    DevBuf<float> moved;                // its particles in tile order (tile_sorted_copy)
 };
 
 }  // namespace aw
@@ -271,6 +272,12 @@ bool tile_sort_onepass(aw_ctx& c, const aw_particles& src, const aw_particles& d
 // in tile order, off[ntiles + 1] (one-pass counting sort when the per-tile
 // counters fit LDS, else the radix sort of tile keys).
 void bin_tiles(aw_ctx& c, const aw_particles& p, int32_t* perm, int32_t* off, hipStream_t s);
+
+// p copied in stable tile order into the context's scratch (x, y and w only, or
+// all of it), the offsets in c.sort.bin_off.  False, and nothing done, where
+// the one-pass sort does not apply or the copy has no room.
+bool tile_sorted_copy(aw_ctx& c, const aw_particles& p, bool positions_only, aw_particles& out,
+                      hipStream_t s);
 
 // Esirkepov current (esirkepov.hip).  Optional inputs: fixed scale bounds the
 // caller guarantees, in place of a bound pass over the particles; the tile

@@ -924,10 +924,15 @@ int dcu_part_capacity() { return 2 * 256; }
 // scales come from the measured max |w| and max |u|.  The push gathers from
 // the packed grid.
 
-static void bin_particles(aw_ctx& c, const aw_particles& p, hipStream_t s) {
+// q = p in tile order and no permutation, or p itself and the bins of its tiles
+static const int32_t* bin_particles(aw_ctx& c, const aw_particles& p, aw_particles& q,
+                                    hipStream_t s) {
+    if (tile_sorted_copy(c, p, false, q, s)) return nullptr;
+    q = p;
     c.sort.bin_off.reserve((size_t)c.ntiles + 1);
     c.sort.bin_perm.reserve((size_t)std::max<int64_t>(1, p.n));
     bin_tiles(c, p, c.sort.bin_perm.get(), c.sort.bin_off.get(), s);
+    return c.sort.bin_perm.get();
 }
 
 static void measure_scales(aw_ctx& c, const aw_particles& p, double qm, hipStream_t s) {
@@ -954,9 +959,10 @@ void deposit_rho_j_amu(aw_ctx& c, const aw_particles& p, double qm, float* const
     EmScratch& e = c.em;
     e.acc.reserve((size_t)(8 * nc));
     AW_HIP(hipMemsetAsync(e.acc.get(), 0, (size_t)(8 * nc) * sizeof(unsigned long long), s));
-    bin_particles(c, p, s);
+    aw_particles q;
+    const int32_t* idx = bin_particles(c, p, q, s);
     measure_scales(c, p, qm, s);
-    em_moments(c, p, c.sort.bin_off.get(), c.sort.bin_perm.get(), e.acc.get(), e.cq.get(),
+    em_moments(c, q, c.sort.bin_off.get(), idx, e.acc.get(), e.cq.get(),
                em_moments_bpt(c, p.n), nullptr, s, EmBatch{});
     Out8 o{};
     for (int q = 0; q < 8; ++q) o.o[q] = out[q];
@@ -974,12 +980,13 @@ void deposit_dcu(aw_ctx& c, const aw_particles& p, double qm, const float* const
     e.cdcu.reserve(1);
     e.fpart.reserve(512);
     AW_HIP(hipMemsetAsync(e.acc.get(), 0, (size_t)(3 * nc) * sizeof(unsigned long long), s));
-    bin_particles(c, p, s);
+    aw_particles q;
+    const int32_t* idx = bin_particles(c, p, q, s);
     measure_scales(c, p, qm, s);
     const double mult = p.w ? 1.0 : p.w_uniform;
     dcu_scale(F, nc, e.fpart.get(), 0.0, qm * qm * mult / (c.g.dx * c.g.dy), 0.0, e.dv.get(),
               e.cdcu.get(), e.inv.get() + 8, s, 1, 0, 0, 0);
-    em_dcu(c, p, c.sort.bin_off.get(), c.sort.bin_perm.get(), F, e.acc.get(), e.cdcu.get(),
+    em_dcu(c, q, c.sort.bin_off.get(), idx, F, e.acc.get(), e.cdcu.get(),
            tile_bpt(c, p.n), nullptr, s, EmBatch{});
     Out8 o{};
     for (int q = 0; q < 3; ++q) o.o[q] = out[q];

@@ -296,12 +296,20 @@ void deposit_rho_fixed(aw_ctx& c, const aw_particles& p, double qm, int policy,
             t.idx = nullptr;
             t.apron = c.apron;
         } else {
-            // Particles::build_tile_bins (include/pic/particles.hpp:632-671)
-            c.sort.bin_off.reserve((size_t)c.ntiles + 1);
-            c.sort.bin_perm.reserve((size_t)std::max<int64_t>(1, p.n));
-            bin_tiles(c, p, c.sort.bin_perm.get(), c.sort.bin_off.get(), s);
+            // Particles::build_tile_bins (include/pic/particles.hpp:632-671),
+            // the positions with them where they can be copied
+            aw_particles q;
+            if (tile_sorted_copy(c, p, true, q, s)) {
+                a.x = q.x;
+                a.y = q.y;
+                a.w = q.w;
+            } else {
+                c.sort.bin_off.reserve((size_t)c.ntiles + 1);
+                c.sort.bin_perm.reserve((size_t)std::max<int64_t>(1, p.n));
+                bin_tiles(c, p, c.sort.bin_perm.get(), c.sort.bin_off.get(), s);
+                t.idx = c.sort.bin_perm.get();
+            }
             t.off = c.sort.bin_off.get();
-            t.idx = c.sort.bin_perm.get();
             t.apron = 0;
         }
         t.W = c.tx + 2 * t.apron + 1;
