@@ -286,10 +286,10 @@ bool tile_sorted_copy(aw_ctx& c, const aw_particles& p, bool positions_only, aw_
 // new positions (may alias p.x, p.y).
 struct EskExtra {
     // fixed bounds: (max |w|, max |w uz|) with per-particle deposit weights,
-    // (unused, max |uz|) with w_uniform
+    // (unused, max |uz|) with w_uniform; the caller has set c.jbound to them and
+    // cleared c.jacc
     bool fixed = false;
     int fixed_per_w = 0;
-    bool cleared = false;  // c.jacc cleared and c.jbound set by the caller (fixed)
     float fixed_bound[2] = {0.f, 0.f};
     const int32_t* slice_off = nullptr;
     float *xw = nullptr, *yw = nullptr;

@@ -75,19 +75,6 @@ __global__ void __launch_bounds__(kFinalThreads) esk_bound_final_kernel(const fl
     }
 }
 
-// the accumulators cleared and the fixed bounds written, in one launch
-__global__ void __launch_bounds__(kThreads) esk_begin_kernel(unsigned long long* __restrict__ acc,
-                                                             int64_t n, float f0, float f1,
-                                                             unsigned int* __restrict__ bound) {
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-         i += (int64_t)kThreads * gridDim.x)
-        acc[i] = 0ull;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        bound[0] = __float_as_uint(f0);
-        bound[1] = __float_as_uint(f1);
-    }
-}
-
 __device__ __forceinline__ void write_wrapped(const EskArgs& a, int i) {
     if (a.xw) {
         a.xw[i] = dev::wrap_coord(a.x1[i], (float)a.nx);
@@ -502,12 +489,6 @@ EskArgs setup(aw_ctx& c, const float* x0, const float* y0, const aw_particles& p
         AW_REQUIRE(ex.fixed_bound[0] >= 0.f && ex.fixed_bound[1] >= 0.f &&
                        std::isfinite(ex.fixed_bound[0]) && std::isfinite(ex.fixed_bound[1]),
                    "the current's fixed scale bounds must be finite and non-negative");
-        if (ex.cleared) return a;
-        const int nb = (int)std::min<int64_t>((3 * nc + kThreads - 1) / kThreads,
-                                              8 * std::max(1, c.num_cu));
-        esk_begin_kernel<<<nb, kThreads, 0, s>>>(c.jacc.get(), 3 * nc, ex.fixed_bound[0],
-                                                 ex.fixed_bound[1], c.jbound.get());
-        AW_LAUNCH_CHECK();
         return a;
     }
     const int npart = p.n > 0 ? std::min(blocks_for(p.n), 4 * std::max(1, c.num_cu)) : 0;

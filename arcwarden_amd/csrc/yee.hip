@@ -1406,7 +1406,7 @@ struct aw_maxwell {
             // (wd is clamped to [-8, 1)).  Particles past them set the guard,
             // which synchronize reports.
             wm = weight_max(p);
-            ex.fixed = ex.cleared = true;
+            ex.fixed = true;
             ex.fixed_per_w = rp.deltaf || p.w ? 1 : 0;
             const float wb = rp.deltaf ? 8.f * wm : wm;
             ex.fixed_bound[0] = ex.fixed_per_w ? wb : 0.f;
