@@ -229,14 +229,15 @@ struct EskTiles {
     const int32_t* off;  // ntiles+1, tile bins of the old positions (or of the last sort)
     const int32_t* idx;  // bin permutation (NULL: the particles are in tile order)
     int ntx, tx, ty, A, W, H, bpt;  // A: apron nodes on each side, W = tx + 2A, H = ty + 2A
+    int qslots;                     // slots of a wavefront's move queue (0: none)
 };
 
 // workgroup per (tile, part): the tile's J plus an A-node apron in LDS.  Moves
 // inside their cell are deposited on the spot, the others set aside
 // (MoveQueue): 1.6 M particles on 128x128, 110 us through the bins with the
 // general stencil for all, 25 us from a sorted copy.
-constexpr int kQueueSlots = 64;
-constexpr size_t kQueueLds = (kThreads / 64) * kQueueSlots * MoveQueue::kFloats * sizeof(float);
+constexpr int kQueueSlots = 64;  // a wavefront's, fewer where a large tile leaves less LDS
+constexpr size_t kQueueSlotLds = (kThreads / 64) * MoveQueue::kFloats * sizeof(float);
 template <bool ONE_ROW>
 __global__ void __launch_bounds__(kThreads) esk_tiles_kernel(EskArgs a, EskTiles t,
                                                              unsigned long long* __restrict__ acc) {
@@ -255,8 +256,8 @@ __global__ void __launch_bounds__(kThreads) esk_tiles_kernel(EskArgs a, EskTiles
     const int chunk = (end - beg + t.bpt - 1) / t.bpt;
     const int r0 = beg + part * chunk, r1 = min(end, r0 + chunk);
     MoveQueue queue{reinterpret_cast<float*>(s_j + 3 * R) +
-                        (threadIdx.x >> 6) * kQueueSlots * MoveQueue::kFloats,
-                    kQueueSlots};
+                        (threadIdx.x >> 6) * t.qslots * MoveQueue::kFloats,
+                    t.qslots};
     auto general = [&](float x0, float y0, float x1, float y1, float uz, float w) {
         EskMove m;
         esk_prepare_v(a, x0, y0, x1, y1, uz, a.w ? (double)w : a.w_uniform, kc, m);
@@ -304,9 +305,10 @@ __global__ void __launch_bounds__(kThreads) esk_tiles_kernel(EskArgs a, EskTiles
             }
             write_wrapped(a, i);
         }
-        queue.push(leaves, x0, y0, x1, y1, uz, w, general);
+        if (t.qslots > 0) queue.push(leaves, x0, y0, x1, y1, uz, w, general);
+        else if (leaves) general(x0, y0, x1, y1, uz, w);
     }
-    queue.drain(general);
+    if (t.qslots > 0) queue.drain(general);
     __syncthreads();
     // (row, column) over the three components' 3 H rows, advanced by the
     // stride without dividing
@@ -379,7 +381,12 @@ void deposit_esirkepov(aw_ctx& c, const float* x0, const float* y0, const aw_par
             t.W = c.tx + 2 * t.A;
             t.H = c.ty + 2 * t.A;
             t.bpt = tile_bpt(c, p.n);
-            const size_t sh = (size_t)3 * t.W * t.H * 8 + kQueueLds;
+            size_t sh = (size_t)3 * t.W * t.H * 8;
+            t.qslots = sh < c.lds_per_block
+                           ? (int)std::min<size_t>(kQueueSlots,
+                                                   (c.lds_per_block - sh) / kQueueSlotLds)
+                           : 0;
+            sh += t.qslots * kQueueSlotLds;
             AW_REQUIRE(sh <= c.lds_per_block, "tile apron does not fit LDS");
             launch_one_row(esk_tiles_kernel<true>, esk_tiles_kernel<false>, one_row, c.ntiles * t.bpt, kThreads, sh, s, a, t, acc);
             AW_LAUNCH_CHECK();
@@ -437,7 +444,12 @@ void deposit_esirkepov(aw_ctx& c, const float* x0, const float* y0, const aw_par
             t.W = c.tx + 2 * kApron;
             t.H = c.ty + 2 * kApron;
             t.bpt = tile_bpt(c, p.n);
-            const size_t sh = (size_t)3 * t.W * t.H * 8 + kQueueLds;
+            size_t sh = (size_t)3 * t.W * t.H * 8;
+            t.qslots = sh < c.lds_per_block
+                           ? (int)std::min<size_t>(kQueueSlots,
+                                                   (c.lds_per_block - sh) / kQueueSlotLds)
+                           : 0;
+            sh += t.qslots * kQueueSlotLds;
             launch_one_row(esk_tiles_kernel<true>, esk_tiles_kernel<false>, one_row, c.ntiles * t.bpt, kThreads, sh, s, a, t, acc);
             AW_LAUNCH_CHECK();
         } else {

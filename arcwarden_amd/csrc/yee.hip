@@ -1324,7 +1324,7 @@ struct aw_maxwell {
     // J = the accumulated current after rp.jfilter smoothing passes
     void convert_and_smooth(const esk::EskArgs& e) {
         const Mesh m = mesh();
-        const int fused = std::min(rp.jfilter, kMaxFusedPasses);
+        const int fused = std::clamp(rp.jfilter, 0, kMaxFusedPasses);
         const bool one_row = g.ny == 1;
         const int tx = one_row ? 256 : 32, ty = one_row ? 1 : 8;
         const dim3 grid((g.nx + tx - 1) / tx, (g.ny + ty - 1) / ty, 3);
