@@ -65,11 +65,16 @@ int pair_count(int nq, int ny) { return (nq / 2) * ny + (nq % 2) * ((ny + 1) / 2
 
 int line_ld(int n) { return n + (n >> 3) + 1; }
 
+// Static LDS of the row kernels, beside their lines and twiddles: lines_set's
+// word a wavefront and (kFormEl) the two floats a wavefront of block_max2.
+constexpr int kMaxWaves = 16;
+constexpr size_t kRowsStaticLds = kMaxWaves * (sizeof(int) + 2 * sizeof(float));
+
 // Which of a thread's two lines hold anything, over the workgroup: bit 0 and 1.
 // A line of zeros comes out as zeros, not as the rounding of its partner.
 // Every thread calls it; a barrier is inside.
 __device__ __forceinline__ int lines_set(bool a, bool b) {
-    __shared__ int s_set[16];
+    __shared__ int s_set[kMaxWaves];
     const int m = (__ballot(a) ? 1 : 0) | (__ballot(b) ? 2 : 0);
     if ((threadIdx.x & 63) == 0) s_set[threadIdx.x >> 6] = m;
     __syncthreads();
@@ -539,7 +544,9 @@ void init_own_fft(aw_ctx& c) {
     // 512x512 against 43 / 196 here, while at 256x256 it is behind
     auto pow2 = [](int n) { return (n & (n - 1)) == 0; };
     if (pow2(c.g.nx) && pow2(c.g.ny) && ncell(c) >= (int64_t)1 << 18) return;
-    if (rows_lds(c) > c.lds_per_block || columns_lds(c, 7, 1) > c.lds_per_block) return;
+    if (rows_lds(c) + kRowsStaticLds > c.lds_per_block ||
+        columns_lds(c, 7, 1) > c.lds_per_block)
+        return;
     // both lines' twiddles, then their half-cell phases
     std::vector<double2> tw;
     for (const int n : {c.g.nx, c.g.ny})

@@ -1,8 +1,9 @@
 """GPU tests of the spectral solves on the library's own transforms (fft.hip):
 E of rho, E_L and B of [rho|J], E_T of [dcu|amu] against the same algebra on
 numpy's FP64 transforms, over sides of every factor the transforms have a pass
-for (8, 5, 4, 3, 2, other primes to 61), odd, prime and one-row grids, the
-longest line, and sides that stay with rocFFT (a prime above 61).
+for (5, 4, 3, 2, other primes to 61), odd, prime and one-row grids, the
+longest line, and sides that stay with rocFFT (a prime above 61, a line that
+leaves no LDS for what else its kernels hold).
 
 The library's transforms are FP64 between three FP32 roundings of every value
 (the two half spectra and the result), 2^-24 at most and independent: below
@@ -20,7 +21,7 @@ pytestmark = pytest.mark.gpu
 
 SIDES = [(64, 64), (128, 96), (250, 190), (33, 17), (61, 59), (7, 121), (243, 125), (16, 1),
          (4096, 1), (3001, 1), (1000, 1), (2, 2), (3, 5), (1, 24), (512, 96), (40, 600),
-         (67, 40), (40, 134), (512, 512)]
+         (67, 40), (40, 134), (512, 512), (3150, 1), (3150, 16)]
 
 
 def _own(n):
@@ -96,7 +97,10 @@ def test_solves_match_fp64(solver, nx, ny):
     torch.cuda.synchronize()
     assert np.array_equal(d.cpu().numpy(), src)  # the inputs stay as they are
 
-    own = _own(nx) and _own(ny) and max(nx, ny) <= 4000 and nx * ny < 1 << 18
+    # a line of 3150 takes 163,808 bytes of a workgroup's 163,840 and the row
+    # kernels up to 192 of their own: rocFFT
+    own = (_own(nx) and _own(ny) and max(nx, ny) <= 4000 and nx * ny < 1 << 18
+           and nx != 3150)
     tol = 3.6e-7 if own else 5e-6
     kx, ky, nyq, i, j = _kvec(nx, ny, dx, dy)
     k2 = kx ** 2 + ky ** 2
