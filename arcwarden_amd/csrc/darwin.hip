@@ -334,6 +334,9 @@ __global__ void __launch_bounds__(kThreads) dcu_kernel(EmArgs a) {
 // tile leaves less).
 using esk::MoveQueue;
 constexpr int kQueueSlots = 20;
+// static LDS of the push's kinetic-energy instances, beside the tile and the
+// queue: a double a wavefront
+constexpr size_t kPushStaticLds = (kThreads / 64) * sizeof(double);
 
 struct EmIn {
     float x, y, ux, uy, uz, w;
@@ -828,7 +831,8 @@ int em_push(aw_ctx& c, const aw_particles& p, const int32_t* off, const float* c
     size_t sh = (size_t)a.W * a.H * (8 * 8 + 16 + 8);
     if (esk) {
         constexpr size_t slot = (kThreads / 64) * MoveQueue::kFloats * sizeof(float);
-        const size_t left = c.lds_per_block > sh ? c.lds_per_block - sh : 0;
+        const size_t held = sh + kPushStaticLds;
+        const size_t left = c.lds_per_block > held ? c.lds_per_block - held : 0;
         a.qslots = (int)std::clamp<size_t>(left / slot, 1, kQueueSlots);
         sh += a.qslots * slot;
     }

@@ -83,3 +83,32 @@ def test_darwin_split_deposit_matches_fp64(gpu, oracle, nx, ny, tile, step):
                                w_uniform=s0["w_uniform"])
     for name, r in zip(("Jx", "Jy", "Jz"), ref):
         assert np.linalg.norm(srcs[name] - r) < 1e-6 * np.linalg.norm(r), name
+
+
+@pytest.mark.parametrize("tile_x,tile_y", [(30, 48), (41, 35), (25, 57)])
+def test_darwin_push_on_the_largest_tiles(gpu, tile_x, tile_y):
+    """Tiles whose moments and fields leave LDS for one to six slots of the move
+    queue a wavefront, and whose push also keeps 32 bytes for the kinetic energy
+    of a diagnostics step: the same bits as on 16x16 tiles."""
+    nx, ny, dx = 2 * tile_x, 2 * tile_y, 0.5
+    rp = L.run_params(dt=0.05, qm=-1.0, eps0=1.0, c=8.0, n0=1.0, noisy_load=1, rng_seed=3,
+                      B0=(0.1, 0.0, 0.2), wce=0.2, dump_every=1)
+    sp = [L.species("a", 1.0, 10, (0.5,) * 3, (4.0, -2.0, 0.5))]  # 0.4 cells a step
+    out = []
+    for tx, ty in ((16, 16), (tile_x, tile_y)):
+        sim = Simulation(L.grid(nx, ny, nx * dx, ny * dx), rp, sp,
+                         SimConfig(field_model=L.AW_MODEL_DARWIN,
+                                   current_deposit=L.AW_CURRENT_ESIRKEPOV, tile_x=tx, tile_y=ty,
+                                   sort_every=0, stray_frac=1.0))
+        sim.init()
+        for n in range(3):
+            sim.step(n)
+        srcs, P, hist = sim.sources_all(), sim.particles(), sim.history()
+        sim.close()
+        cols = np.stack([P[k] for k in ("x", "y", "ux", "uy", "uz")])
+        out.append((srcs, cols[:, np.lexsort(cols[::-1])], [h["ke"] for h in hist]))
+    (s0, p0, k0), (s1, p1, k1) = out
+    assert np.array_equal(p0, p1)
+    for name in s0:
+        assert np.array_equal(s0[name], s1[name]), name
+    assert len(k0) == 3 and np.allclose(k0, k1, rtol=1e-12, atol=0)  # FP64 sums, another order
