@@ -261,13 +261,10 @@ struct aw_ensemble {
     }
 
     void convert_and_solve() {
-        // rho^n for every run; rin receives the R2C input copy, strays reset
-        // (on the library's own transforms each size's solve converts for itself)
-        const bool own = std::all_of(groups.begin(), groups.end(), [&](const Group& gr) {
-            return runs[gr.first].ctx->own_fft;
-        });
-        if (!own) fix_to_float_add(acc.get(), rho.get(), nctot, fix_log2, true, stream, true, strays.get(),
-                         rin.get(), (int)runs.size(), rbase.get());
+        // rho^n and E of every run, strays reset.  Each size converts for itself,
+        // on the library's own transforms inside the solve and for rocFFT into
+        // rin before it, so that a run's field does not depend on which other
+        // sizes share the ensemble (a run equals the same run stepped alone).
         // one batched solve per grid size; the sizes touch disjoint buffers
         // (each its own plans, work area and k-space scratch), so they fork
         // onto the side streams and join before the push
@@ -282,11 +279,16 @@ struct aw_ensemble {
             const size_t lane = nside ? g % (nside + 1) : 0;
             aw_ctx& c = *runs[gr.first].ctx;
             const hipStream_t sg = lane ? side[lane - 1] : stream;
-            if (!own) {
+            const int64_t nc = ncell(c);
+            unsigned long long* counter = g == 0 ? strays.get() : nullptr;
+            const int ncounter = g == 0 ? (int)runs.size() : 0;
+            if (!c.own_fft) {
+                fix_to_float_add(acc.get() + gr.cbase, rho.get() + gr.cbase, nc * gr.count,
+                                 fix_log2, true, sg, true, counter, rin.get() + gr.cbase, ncounter,
+                                 rbase.get() + gr.cbase);
                 solve_es_batch(c, gr.count, rin.get() + gr.cbase, E.get() + 2 * gr.cbase, eps0, sg);
                 continue;
             }
-            const int64_t nc = ncell(c);
             SpecSrc in;
             in.acc = acc.get() + gr.cbase;
             in.acc_rs = nc;
@@ -295,10 +297,8 @@ struct aw_ensemble {
             in.inv0 = std::ldexp(1.0, -fix_log2);
             in.base = rbase.get() + gr.cbase;
             in.base_cell = 1;
-            if (g == 0) {
-                in.counter = strays.get();
-                in.ncounter = (int)runs.size();
-            }
+            in.counter = counter;
+            in.ncounter = ncounter;
             SpecDst out;
             out.out = E.get() + 2 * gr.cbase;
             out.out1 = out.out + nc;

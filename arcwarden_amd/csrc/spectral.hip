@@ -180,17 +180,14 @@ void fft_exec(aw_ctx& c, rocfft_plan plan, void* in, void* out, hipStream_t s) {
 }
 
 namespace {
-// runs of FP32 rho -> (Ex, Ey), rs apart, on the library's own transforms
-void own_es(aw_ctx& c, const float* rho, float* Ex, float* Ey, int64_t rs, double eps0, int runs,
-            hipStream_t s) {
+// FP32 rho -> Ex, Ey on the library's own transforms
+void own_es(aw_ctx& c, const float* rho, float* Ex, float* Ey, double eps0, hipStream_t s) {
     SpecSrc in;
     in.in = rho;
-    in.in_rs = ncell(c);
     SpecDst out;
     out.out = Ex;
     out.out1 = Ey;
-    out.out_rs = rs;
-    spec_solve_es(c, in, out, eps0, runs, s);
+    spec_solve_es(c, in, out, eps0, 1, s);
 }
 
 // nin contiguous FP32 grids a run in, nout out
@@ -297,13 +294,10 @@ void enable_batch_fft(aw_ctx& c, int batch) {
 }
 
 // rho_in: B grids [B][ny][nx] (rocFFT may overwrite them); E2B: [B][Ex|Ey].
+// Only where the solves are rocFFT's (not own_fft).
 void solve_es_batch(aw_ctx& c, int batch, float* rho_in, float* E2B, double eps0,
                     hipStream_t s) {
-    AW_REQUIRE(c.fft_batch == batch, "batched plans not prepared for this batch");
-    if (c.own_fft) {
-        own_es(c, rho_in, E2B, E2B + ncell(c), 2 * ncell(c), eps0, batch, s);
-        return;
-    }
+    AW_REQUIRE(c.fft_batch == batch && !c.own_fft, "batched plans not prepared for this batch");
     const int64_t nk = nkmodes(c);
     c.ktmp.reserve((size_t)6 * nk * batch);
     float2* rk = reinterpret_cast<float2*>(c.ktmp.get());
@@ -318,7 +312,7 @@ void solve_es_batch(aw_ctx& c, int batch, float* rho_in, float* E2B, double eps0
 
 void solve_es_contig(aw_ctx& c, const float* rho, float* E2, double eps0, hipStream_t s) {
     if (c.own_fft) {
-        own_es(c, rho, E2, E2 + ncell(c), 0, eps0, 1, s);
+        own_es(c, rho, E2, E2 + ncell(c), eps0, s);
         return;
     }
     const int64_t nk = nkmodes(c);
@@ -490,7 +484,7 @@ void solve_darwin_et(aw_ctx& c, const float* src7, float* out3, double eps0, dou
 // General form with separate output buffers.
 void solve_es(aw_ctx& c, const float* rho, float* Ex, float* Ey, double eps0, hipStream_t s) {
     if (c.own_fft) {
-        own_es(c, rho, Ex, Ey, 0, eps0, 1, s);
+        own_es(c, rho, Ex, Ey, eps0, s);
         return;
     }
     const int64_t nk = nkmodes(c);

@@ -90,6 +90,30 @@ def test_five_grid_sizes_share_the_solve_streams(gpu, graph):
     ens.close()
 
 
+# 67 and 134 stay with rocFFT, the others take the library's own transforms
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("sides", [(32, 67, 48, 32), (96, 67, 134, 67), (24, 134, 40, 67, 16)])
+def test_sizes_of_either_transform_match_single_runs(gpu, sides, graph):
+    """A run equals the same run stepped alone bit for bit, whichever transform
+    its own size and the other sizes of the ensemble take."""
+    runs = [two_beam_run(sd, 16, 0.02, 0.2 + 0.01 * i, seed=600 + i) for i, sd in enumerate(sides)]
+    nsteps = 9
+    ens = Ensemble(runs, SimConfig(sort_every=4), graph=graph)
+    ens.init()
+    assert ens.info()["ngroups"] == len(set(sides))
+    ens.run(0, nsteps)
+    for i, r in enumerate(runs):
+        s = Simulation(r.grid, r.rp, r.species, SimConfig(has_b0=False, sort_every=4))
+        s.init()
+        s.run(nsteps)
+        assert np.array_equal(ens.rho(i), s.rho()), i
+        f, fs = ens.fields(i), s.fields()
+        assert np.array_equal(f["Ex"], fs["Ex"]) and np.array_equal(f["Ey"], fs["Ey"]), i
+        assert np.array_equal(_multiset(ens.particles(i)), _multiset(s.particles())), i
+        s.close()
+    ens.close()
+
+
 @pytest.mark.parametrize("graph", [False, True])
 def test_stray_sort_is_per_run(gpu, graph):
     """Only the run whose particles strayed beyond the threshold is re-sorted
