@@ -963,9 +963,9 @@ void deposit_rho_j_amu(aw_ctx& c, const aw_particles& p, double qm, float* const
     EmScratch& e = c.em;
     e.acc.reserve((size_t)(8 * nc));
     AW_HIP(hipMemsetAsync(e.acc.get(), 0, (size_t)(8 * nc) * sizeof(unsigned long long), s));
+    measure_scales(c, p, qm, s);  // its scratch before the copy of the particles
     aw_particles q;
     const int32_t* idx = bin_particles(c, p, q, s);
-    measure_scales(c, p, qm, s);
     em_moments(c, q, c.sort.bin_off.get(), idx, e.acc.get(), e.cq.get(),
                em_moments_bpt(c, p.n), nullptr, s, EmBatch{});
     Out8 o{};
@@ -984,9 +984,9 @@ void deposit_dcu(aw_ctx& c, const aw_particles& p, double qm, const float* const
     e.cdcu.reserve(1);
     e.fpart.reserve(512);
     AW_HIP(hipMemsetAsync(e.acc.get(), 0, (size_t)(3 * nc) * sizeof(unsigned long long), s));
+    measure_scales(c, p, qm, s);  // its scratch before the copy of the particles
     aw_particles q;
     const int32_t* idx = bin_particles(c, p, q, s);
-    measure_scales(c, p, qm, s);
     const double mult = p.w ? 1.0 : p.w_uniform;
     dcu_scale(F, nc, e.fpart.get(), 0.0, qm * qm * mult / (c.g.dx * c.g.dy), 0.0, e.dv.get(),
               e.cdcu.get(), e.inv.get() + 8, s, 1, 0, 0, 0);

@@ -715,6 +715,21 @@ void stable_sort_keys(aw_ctx& c, int64_t n, uint32_t nkeys, int32_t* perm, int32
     }
 }
 
+// Chunks of a one-pass sort of n particles, and the scratch it takes.
+struct TsPlan {
+    int rounds, nchunks, nblk;
+};
+static TsPlan ts_reserve(aw_ctx& c, int64_t n) {
+    TsPlan p;
+    p.rounds = ts_rounds(n, c.ntiles);
+    p.nchunks = (int)((n + kTsWave * p.rounds - 1) / (kTsWave * p.rounds));
+    p.nblk = (p.nchunks + kTsColBlock - 1) / kTsColBlock;
+    const size_t nt = (size_t)c.ntiles;
+    c.sort.table.reserve(nt * p.nchunks);
+    c.sort.colsum.reserve((size_t)p.nblk * nt + nt + 1);
+    return p;
+}
+
 // Stable tile sort src -> dst in one pass (see ts_* kernels).  Returns false
 // when the per-tile LDS tables do not fit (caller uses the radix path).
 bool tile_sort_onepass(aw_ctx& c, const aw_particles& src, const aw_particles& dst, int32_t* off,
@@ -727,22 +742,17 @@ bool tile_sort_onepass(aw_ctx& c, const aw_particles& src, const aw_particles& d
         AW_HIP(hipMemsetAsync(off, 0, ((size_t)c.ntiles + 1) * sizeof(int32_t), s));
         return true;
     }
-    const int rounds = ts_rounds(n, c.ntiles);
-    const int nchunks = (int)(((int64_t)n + kTsWave * rounds - 1) / (kTsWave * rounds));
+    const auto [rounds, nchunks, nblk] = ts_reserve(c, n);
     int tbits = 0;
     while ((1 << tbits) < c.ntiles) ++tbits;
-    c.sort.table.reserve((size_t)c.ntiles * nchunks);
     AW_REQUIRE(c.g.nx < (1 << 24) && c.g.ny < (1 << 24), "grid sides must be below 2^24");
     const TileMap tm{c.g.nx, c.g.ny, c.tx, c.ty, c.ntx, 1.0f / (float)c.tx, 1.0f / (float)c.ty};
     ts_hist_kernel<<<nchunks, kTsHistThreads, lds, s>>>(src.x, src.y, n, tm, c.ntiles, rounds,
                                                         c.sort.table.get());
     AW_LAUNCH_CHECK();
     // offsets of the chunk-major table (see ts_colsum_kernel)
-    const int nblk = (nchunks + kTsColBlock - 1) / kTsColBlock;
-    const size_t nt = (size_t)c.ntiles;
-    c.sort.colsum.reserve((size_t)nblk * nt + nt + 1);
     uint32_t* bsum = c.sort.colsum.get();
-    uint32_t* tbase = bsum + (size_t)nblk * nt;  // tile totals, scanned into tile bases
+    uint32_t* tbase = bsum + (size_t)nblk * c.ntiles;  // tile totals, scanned into tile bases
     const dim3 cg(blocks_for((int64_t)c.ntiles), nblk);
     ts_colsum_kernel<<<cg, kThreads, 0, s>>>(c.sort.table.get(), nchunks, c.ntiles, bsum);
     AW_LAUNCH_CHECK();
@@ -778,8 +788,10 @@ bool tile_sorted_copy(aw_ctx& c, const aw_particles& p, bool positions_only, aw_
     if ((size_t)c.ntiles * 4 > c.lds_per_block || p.n == 0) return false;
     const size_t n = (size_t)p.n;
     const int nf = (positions_only ? 2 : 5) + (p.w ? 1 : 0);
+    // what the bins take too comes first, so that a copy that fits leaves room for it
+    c.sort.bin_off.reserve((size_t)c.ntiles + 1);
+    (void)ts_reserve(c, p.n);
     try {
-        c.sort.bin_off.reserve((size_t)c.ntiles + 1);
         c.sort.moved.reserve((size_t)nf * n);
     } catch (const AwError&) {  // no room for a copy: the caller takes the bins
         (void)hipGetLastError();

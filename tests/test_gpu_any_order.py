@@ -1,8 +1,9 @@
 """GPU tests of the operators on particles in no order, at the sizes where
 their dispatch or their indexing changes: the tile sort's one-workgroup and
 general offset scans, waves that name more tiles than are matched one by one,
-and the gathers across the right and upper edges.  Integer results and the
-FP32 pushes are compared bit for bit."""
+the binned deposits on a sorted copy and through the permutation, and the
+gathers across the right and upper edges.  Integer results and the FP32 pushes
+are compared bit for bit."""
 import ctypes as C
 
 import numpy as np
@@ -98,3 +99,50 @@ def test_push_boris_em_edges(gpu, oracle, nx, ny, n):
         got = p.numpy()
     for k in ("x", "y", "ux", "uy", "uz"):
         assert np.array_equal(got[k], ref[k]), k
+
+
+def _binned_deposits(ctx, st, w, x1, y1, Fd, nc):
+    """rho, the Darwin moments, dcu and the Esirkepov current, binned."""
+    wu = 0.0 if w is not None else 0.25
+    p = DevParticles(st, w=w, w_uniform=wu)
+    moved = DevParticles({**st, "x": x1, "y": y1}, w=w, w_uniform=wu)
+    f = L.AwFields()
+    for name, t in zip(("Ex", "Ey", "Ez", "Bx", "By", "Bz"), Fd):
+        setattr(f, name, t.data_ptr())
+    out = [torch.zeros(nc, dtype=torch.float32, device="cuda") for _ in range(15)]
+    src = L.AwSources()
+    for name, t in zip(("rho", "Jx", "Jy", "Jz", "amu0", "amu1", "amu2", "amu3", "dcux", "dcuy",
+                        "dcuz"), out):
+        setattr(src, name, t.data_ptr())
+    L.call("aw_deposit_rho_j_amu", ctx.h, C.byref(p.struct()), -1.0, C.byref(src), stream())
+    L.call("aw_deposit_dcu", ctx.h, C.byref(p.struct()), -1.0, C.byref(f), C.byref(src), stream())
+    L.call("aw_deposit_rho", ctx.h, C.byref(p.struct()), -1.0, L.AW_DEPOSIT_BINNED,
+           out[11].data_ptr(), stream())
+    L.call("aw_deposit_esirkepov", ctx.h, p.t["x"].data_ptr(), p.t["y"].data_ptr(),
+           C.byref(moved.struct()), -1.0, 0.1, L.AW_DEPOSIT_BINNED,
+           *(t.data_ptr() for t in out[12:]), stream())
+    return [host(t) for t in out]
+
+
+# tiles of 2x2 on 512x512: 65536, whose counters do not fit LDS, so the
+# particles are read through the radix sort's permutation; 16x16: from a copy
+# in tile order.  The sums are integers: the same bits.
+@pytest.mark.parametrize("per_w", [False, True])
+def test_binned_deposits_copy_and_permutation(gpu, per_w):
+    nx = ny = 512
+    n = 150_003
+    rng = np.random.default_rng(17 + per_w)
+    st = _edge_particles(rng, nx, ny, n)
+    x1 = np.mod(st["x"] + rng.uniform(-0.9, 0.9, n).astype(np.float32), np.float32(nx))
+    y1 = np.mod(st["y"] + rng.uniform(-0.9, 0.9, n).astype(np.float32), np.float32(ny))
+    x1[x1 >= nx], y1[y1 >= ny] = 0, 0
+    w = rng.uniform(0.1, 0.4, n).astype(np.float32) if per_w else None
+    g = L.grid(nx, ny, 0.5 * nx, 0.5 * ny)
+    Fd = [dev(a.ravel()) for a in _fields(rng, 6, nx, ny)]
+    got = []
+    for t in (16, 2):
+        with Ctx(g, t, t) as ctx:
+            assert (ctx.ntiles > 40960) == (t == 2)
+            got.append(_binned_deposits(ctx, st, w, x1, y1, Fd, nx * ny))
+    for q, (a, b) in enumerate(zip(*got)):
+        assert np.abs(a).max() > 0 and np.array_equal(a, b), q
