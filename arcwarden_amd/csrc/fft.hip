@@ -508,7 +508,10 @@ void solve(aw_ctx& c, const SpecSrc& in, const SpecDst& out, const Op& op, int r
     constexpr int NM = std::max(Op::kIn, Op::kOut);
     const int64_t nk = nkmodes(c);
     const int ny = c.g.ny;
-    c.ktmp.reserve((size_t)2 * (Op::kIn + Op::kOut) * nk * runs);
+    // either Darwin solve allocates for both, so that the second allocates nothing
+    // (a caller may capture it after a first call of the other)
+    constexpr int kGrids = std::max(Op::kIn + Op::kOut, Op::kIn > 2 ? OpEt::kIn + OpEt::kOut : 0);
+    c.ktmp.reserve((size_t)2 * kGrids * nk * runs);
     float2* kin = reinterpret_cast<float2*>(c.ktmp.get());
     float2* kout = kin + (size_t)Op::kIn * nk * runs;
     const int rt = threads_for(c.g.nx / kAhead, 1024);

@@ -125,3 +125,41 @@ def test_solves_match_fp64(solver, nx, ny):
     J[0], J[1] = J[0] - kx * kd, J[1] - ky * kd
     G = np.where(on, 1.0 / (eps0 * c * c * safe + n0), 0)
     _check(et.cpu().numpy(), _inverse([-G * v for v in J], nx, ny), tol)
+
+
+def test_darwin_solves_captured_after_the_first(solver):
+    """Once one Darwin solve has run, a graph captures both (nothing is left to
+    allocate); every replay equals the eager result of the same inputs."""
+    nx, ny = 96, 50
+    ctx = solver(nx, ny, 0.5, 0.4)
+    rng = np.random.default_rng(5)
+    d = torch.zeros(11, ny, nx, device="cuda")
+    elb, et = torch.zeros(5, ny, nx, device="cuda"), torch.zeros(3, ny, nx, device="cuda")
+    b0 = (C.c_float * 3)(0.3, -0.2, 0.1)
+
+    def el_b(out):
+        L.call("aw_solve_darwin_el_b", ctx, d.data_ptr(), out.data_ptr(), 1.0, 7.0, b0,
+               C.c_void_p(torch.cuda.current_stream().cuda_stream))
+
+    def e_t(out):
+        L.call("aw_solve_darwin_et", ctx, d[4].data_ptr(), out.data_ptr(), 1.0, 7.0, 0.9,
+               C.c_void_p(torch.cuda.current_stream().cuda_stream))
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        el_b(elb)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        el_b(elb)
+        e_t(et)
+    for _ in range(3):
+        d.copy_(torch.from_numpy(rng.normal(size=(11, ny, nx)).astype(np.float32)))
+        ref_b, ref_t = torch.zeros_like(elb), torch.zeros_like(et)
+        el_b(ref_b)
+        e_t(ref_t)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(elb, ref_b) and torch.equal(et, ref_t)
+        assert float(et.abs().max()) > 0
