@@ -322,11 +322,11 @@ long long rho_baseline(double qm, double density, int scale_log2);
 void deposit_rho_fixed(aw_ctx& c, const aw_particles& p, double qm, int policy,
                        const int32_t* sorted_off, hipStream_t s,
                        unsigned long long* acc = nullptr);
-int tile_bpt(const aw_ctx& c, int64_t n);
-int balanced_bpt(const aw_ctx& c, int64_t n, size_t lds, int waves, int fixed);
+int tile_bpt(const aw_ctx& c, int64_t n, int runs = 1);
+int balanced_bpt(const aw_ctx& c, int64_t n, size_t lds, int waves, int fixed, int runs = 1);
 // Darwin kernels (darwin.hip): their workgroups per tile unless configured
-int em_push_bpt(const aw_ctx& c, int64_t n);
-int em_moments_bpt(const aw_ctx& c, int64_t n);
+int em_push_bpt(const aw_ctx& c, int64_t n, int runs);
+int em_moments_bpt(const aw_ctx& c, int64_t n, int runs);
 
 // The external pump wave (include/pic/pump.hpp:34-47).
 struct PumpArgs {

@@ -43,7 +43,6 @@ size_t ke_stage_capacity(size_t nke);
 int reduce_partial_capacity();
 int reduce_grid_offset();
 int reduce_out_offset();
-int tile_bpt(const aw_ctx& c, int64_t n);
 bool uz_evolves(const aw_run_params& rp, bool has_b0);
 void enable_em_fft(aw_ctx& c);
 void solve_darwin_elb(aw_ctx& c, const float* src4, float* out5, double eps0, double cl,
@@ -543,9 +542,9 @@ struct aw_sim {
             bpt = tile_bpt(*ctx, n);
             return;
         }
-        bpt = em_push_bpt(*ctx, n);
+        bpt = em_push_bpt(*ctx, n, runs);
         bpt_dcu = tile_bpt(*ctx, n);
-        bpt_moments = em_moments_bpt(*ctx, n);
+        bpt_moments = em_moments_bpt(*ctx, n, runs);
     }
 
     // Tile geometry and workgroups per tile of the particle kernels.

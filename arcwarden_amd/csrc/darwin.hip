@@ -722,7 +722,6 @@ __global__ void convert_add_kernel(const unsigned long long* __restrict__ acc, O
 
 // ---- host side ------------------------------------------------------------------------
 
-int tile_bpt(const aw_ctx& c, int64_t n);
 
 static EmArgs em_args(aw_ctx& c, const aw_particles& p, const int32_t* off, const int32_t* idx,
                       const float* const* F, unsigned long long* acc, const float* cq,
@@ -772,11 +771,11 @@ static size_t tile_nodes(const aw_ctx& c) {
     return (size_t)(c.tx + 2 * c.apron + 1) * (c.ty + 2 * c.apron + 1);
 }
 // the moments' and the push's accumulators (and fields) per node of the tile
-int em_push_bpt(const aw_ctx& c, int64_t n) {
-    return balanced_bpt(c, n, tile_nodes(c) * 88, 4, 3);
+int em_push_bpt(const aw_ctx& c, int64_t n, int runs) {
+    return balanced_bpt(c, n, tile_nodes(c) * 88, 4, 3, runs);
 }
-int em_moments_bpt(const aw_ctx& c, int64_t n) {
-    return balanced_bpt(c, n, tile_nodes(c) * 64, 8, 3);
+int em_moments_bpt(const aw_ctx& c, int64_t n, int runs) {
+    return balanced_bpt(c, n, tile_nodes(c) * 64, 8, 3, runs);
 }
 
 static void set_batch(EmArgs& a, const EmBatch& b) {
@@ -967,7 +966,7 @@ void deposit_rho_j_amu(aw_ctx& c, const aw_particles& p, double qm, float* const
     aw_particles q;
     const int32_t* idx = bin_particles(c, p, q, s);
     em_moments(c, q, c.sort.bin_off.get(), idx, e.acc.get(), e.cq.get(),
-               em_moments_bpt(c, p.n), nullptr, s, EmBatch{});
+               em_moments_bpt(c, p.n, 1), nullptr, s, EmBatch{});
     Out8 o{};
     for (int q = 0; q < 8; ++q) o.o[q] = out[q];
     convert_add_kernel<<<blocks_for(nc), kThreads, 0, s>>>(e.acc.get(), o, (int)nc, 8, e.inv.get());

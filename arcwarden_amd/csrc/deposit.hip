@@ -203,7 +203,7 @@ void deposit_rho_acc(const aw_grid& g, const aw_particles& p, double qm, int pol
     }
 }
 
-int tile_bpt(const aw_ctx& c, int64_t n) {
+int tile_bpt(const aw_ctx& c, int64_t n, int runs) {
     // about 2048 particles (8 per lane) per workgroup: enough to amortise the
     // tile load and flush, few enough that the grid holds many workgroups per
     // CU and the tail of the launch stays short
@@ -212,7 +212,7 @@ int tile_bpt(const aw_ctx& c, int64_t n) {
     // small grids: keep >= 4 workgroups per CU while each keeps >= 1 particle
     // per lane
     const int64_t want = 4ll * std::max(1, c.num_cu);
-    while (bpt < 64 && (int64_t)c.ntiles * bpt < want && per_tile / (2 * bpt) >= kThreads)
+    while (bpt < 64 && (int64_t)c.ntiles * runs * bpt < want && per_tile / (2 * bpt) >= kThreads)
         bpt *= 2;
     return bpt;
 }
@@ -224,20 +224,23 @@ int tile_bpt(const aw_ctx& c, int64_t n) {
 // rounds wastes most of one; past six rounds the workgroups finish out of step
 // and tile_bpt's share stands (156 M Yee particles: 1632 us, 1657 us with as few
 // workgroups as this would take).  lds: a workgroup's LDS; waves: the kernel's
-// waves per SIMD.  The relativistic Yee push of 0.98 M particles on 250x130 went
-// from 1152 workgroups to 1008 and from 38.9 to 34.3 us, the Darwin moments of
-// 1.6 M on 128x128 from 1664 to 1280 and from 96 to 61 us.
-int balanced_bpt(const aw_ctx& c, int64_t n, size_t lds, int waves, int fixed) {
+// waves per SIMD; runs: of a batch, n particles each, all in one launch.  The
+// relativistic Yee push of 0.98 M particles on 250x130 went from 1152
+// workgroups to 1008 and from 38.9 to 34.3 us, the Darwin moments of 1.6 M on
+// 128x128 from 1664 to 1280 and from 96 to 61 us.  With the runs counted, a
+// Darwin batch of 16 runs of 64x64 x 64 takes 377 us a step instead of 668.
+int balanced_bpt(const aw_ctx& c, int64_t n, size_t lds, int waves, int fixed, int runs) {
     const double per_tile = (double)n / std::max(1, c.ntiles);
     const int per_cu = (int)std::clamp<size_t>(c.lds_per_block / std::max<size_t>(1, lds), 1,
                                                (size_t)waves);
     const double slots = (double)per_cu * std::max(1, c.num_cu);
-    int best = tile_bpt(c, n);
-    if ((double)c.ntiles * best > 6.0 * slots) return best;
+    int best = tile_bpt(c, n, runs);
+    const double tiles = (double)c.ntiles * runs;
+    if (tiles * best > 6.0 * slots) return best;
     double best_cost = 0.0;
     for (int b = 1; b <= 64; ++b) {
         if (b > 1 && per_tile / b < kThreads) break;
-        const double rounds = std::ceil((double)c.ntiles * b / slots);
+        const double rounds = std::ceil(tiles * b / slots);
         const double cost = rounds * (fixed + std::ceil(per_tile / b / kThreads));
         if (b == 1 || cost < best_cost) {
             best = b;

@@ -348,7 +348,6 @@ __global__ void __launch_bounds__(kThreads) esk_convert_kernel(EskArgs a,
 
 }  // namespace
 
-int tile_bpt(const aw_ctx& c, int64_t n);
 
 namespace {
 // the one-row (ny = 1) instance of a kernel, or the general one

@@ -320,7 +320,6 @@ push_deposit_multi_kernel(const RunSlot* __restrict__ runs, const int32_t* __res
 
 }  // namespace
 
-int tile_bpt(const aw_ctx& c, int64_t n);
 bool uz_evolves(const aw_run_params& rp, bool has_b0);
 
 void push_es(aw_ctx& c, const aw_particles& p, const float* Ex, const float* Ey,

@@ -34,7 +34,6 @@
 
 namespace aw {
 
-int tile_bpt(const aw_ctx& c, int64_t n);
 
 namespace {
 
