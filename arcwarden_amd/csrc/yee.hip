@@ -671,18 +671,24 @@ yee_push_esk_tiles_kernel(PushArgs a, Mesh m, aw_run_params rp, PushTiles t, esk
 // wavefront then sums its quanta across the lanes and one lane adds them.
 // 3.4 M delta-f particles on 5000 cells: push 66 us + deposit 46 us before,
 // 93 us.
+// The instance with the pump or the relativistic push has 512 threads: at 1024
+// it spilled 37 registers, which cost more than the wavefronts hid on lines of
+// up to a million particles (relativistic, 4000 cells x 200: 45.5 us a step
+// against 41.8, 256 x 50: 26.6 against 22.5; 5000 x 676: 92 against 100).
 constexpr int kRowThreads = 1024;
+constexpr int row_threads(bool nopr) { return nopr ? kRowThreads : 512; }
 
 template <bool PLAIN, bool NOPR>
-__global__ void __launch_bounds__(kRowThreads)
+__global__ void __launch_bounds__(row_threads(PLAIN || NOPR))
 yee_push_esk_row_kernel(PushArgs a, Mesh m, aw_run_params rp, esk::EskArgs e, int qslots,
                         unsigned long long* __restrict__ acc) {
+    constexpr int kThr = row_threads(PLAIN || NOPR);
     extern __shared__ unsigned long long s_mem[];
     const int nc = m.nx;
     MoveQueue queue{reinterpret_cast<float*>(s_mem + 3 * nc) +
                         (threadIdx.x >> 6) * qslots * MoveQueue::kFloats,
                     qslots};
-    for (int c = threadIdx.x; c < 3 * nc; c += kRowThreads) s_mem[c] = 0ull;
+    for (int c = threadIdx.x; c < 3 * nc; c += kThr) s_mem[c] = 0ull;
     __syncthreads();
     const MeshGather gat{m};
     double kc[3];
@@ -697,8 +703,8 @@ yee_push_esk_row_kernel(PushArgs a, Mesh m, aw_run_params rp, esk::EskArgs e, in
             atomicAdd(&s_mem[q * nc + gx[k - 1]], v);
         });
     };
-    const int64_t stride = (int64_t)kRowThreads * gridDim.x;
-    for (int64_t base = (int64_t)blockIdx.x * kRowThreads; base < a.n; base += stride) {
+    const int64_t stride = (int64_t)kThr * gridDim.x;
+    for (int64_t base = (int64_t)blockIdx.x * kThr; base < a.n; base += stride) {
         const int64_t t = base + threadIdx.x;
         bool leaves = false;
         int cell = -1;
@@ -752,7 +758,7 @@ yee_push_esk_row_kernel(PushArgs a, Mesh m, aw_run_params rp, esk::EskArgs e, in
     }
     queue.drain(general);
     __syncthreads();
-    for (int c = threadIdx.x; c < 3 * nc; c += kRowThreads) {
+    for (int c = threadIdx.x; c < 3 * nc; c += kThr) {
         const unsigned long long v = s_mem[c];
         if (v) atomicAdd(&acc[c], v);
     }
@@ -1527,10 +1533,11 @@ struct aw_maxwell {
                                 ? yee_push_esk_row_kernel<true, false>
                             : nopr ? yee_push_esk_row_kernel<false, true>
                                    : yee_push_esk_row_kernel<false, false>;
-                const int nb1 = (int)std::min<int64_t>((p.n + kRowThreads - 1) / kRowThreads,
+                const int nt = row_threads(nopr);
+                const int nb1 = (int)std::min<int64_t>((p.n + nt - 1) / nt,
                                                        std::max(1, ctx->num_cu));
-                kern<<<nb1, kRowThreads, row_lds + slots * kSlot, stream>>>(a, m, rp, e, slots,
-                                                                           ctx->jacc.get());
+                kern<<<nb1, nt, row_lds + slots * kSlot, stream>>>(a, m, rp, e, slots,
+                                                                  ctx->jacc.get());
                 AW_LAUNCH_CHECK();
                 convert_and_smooth(e);
             } else {

@@ -4,7 +4,8 @@
   (FP32, same operation sequence), the current of the move within 1e-6 of
   the FP64 Esirkepov restatement, across B0 orientations, the relativistic
   push, delta-f weights (three precisions), the mirror background on a
-  one-row grid, reflecting walls and the pump, and the current smoothing in
+  one-row grid, reflecting walls and the pump (one-row grids too, whose push
+  and current are one kernel), and the current smoothing in
   LDS and in global passes;
 - the tile_sort path (particles kept in tile order, the current deposited
   from the tile slices of the last sort) bit for bit against the unsorted
@@ -67,6 +68,16 @@ CASES = {
     "pump": (48, 12, 0.5, 0.5, dict(B0=(0.4, 0.0, 0.2), pump=1, pump_ex=1e-3, pump_ey=2e-3,
                                     pump_ez=-2e-3, pump_k0=TWO_PI * 3 / 24.0, pump_w0=0.15,
                                     pump_trmp=0.5, pump_toff=100.0)),
+    # one row at 16 particles a cell or more: the push and the current in one kernel
+    "relativistic_one_row": (300, 1, 0.5, 0.5, dict(B0=(0.2, 0.0, 0.4), rel=1)),
+    "pump_one_row": (257, 1, 0.5, 0.5, dict(B0=(0.4, 0.0, 0.2), pump=1, pump_ex=1e-3,
+                                            pump_ey=2e-3, pump_ez=-2e-3,
+                                            pump_k0=TWO_PI * 3 / 128.5, pump_w0=0.15,
+                                            pump_trmp=0.5, pump_toff=100.0)),
+    "walls_deltaf_pump_rel_one_row": (128, 1, 0.5, 0.5, dict(
+        B0=(0.5, 0.0, 0.0), rel=1, bnd_x=2, bnd_nd=6, bnd_numax=0.5, deltaf=1, df_tpar=0.01,
+        df_tperp=0.02, pump=1, pump_ey=2e-3, pump_ez=-2e-3, pump_k0=TWO_PI * 3 / 64.0,
+        pump_w0=0.15, pump_trmp=0.5, pump_toff=100.0)),
 }
 
 
