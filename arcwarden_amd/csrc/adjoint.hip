@@ -795,7 +795,7 @@ struct aw_adjoint {
         } else {
             copy_words(lE0.get(), lEf.get(), (size_t)2 * nc * sizeof(float));
         }
-        if (ctx->own_fft) {
+        if (ctx->own_es) {
             static_assert(kBoundSlots == kSpecSlots && kSlotStride == kSpecSlotStride);
             SpecSrc in;
             in.in = lEf.get();

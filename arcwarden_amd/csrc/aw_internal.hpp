@@ -222,8 +222,9 @@ struct aw_ctx {
     long long rho_base = 0;
     int device = 0, num_cu = 0;
     size_t lds_per_block = 0;
-    // the solves' own transforms (fft.hip) where the grid allows them
-    bool own_fft = false;
+    // the electrostatic and the Darwin solves' own transforms (fft.hip) where
+    // they are ahead of rocFFT
+    bool own_es = false, own_em = false;
     aw::FftLine fx, fy;
     aw::DevBuf<double2> fft_tw;
     rocfft_plan r2c = nullptr, c2r = nullptr, c2r2 = nullptr;
@@ -337,7 +338,7 @@ PumpArgs pump_args(const aw_grid& g, const aw_run_params& rp, double t);
 
 // Solves on the library's own transforms (fft.hip), which fuse the fixed-point
 // conversion before them and the field combination after them; only where
-// own_fft.  A SpecSrc describes the input grids (run r of a batch at r *_rs): fixed-point accumulators acc[q], converted as convert_multi does
+// own_es (spec_solve_es, _adj) or own_em (_elb, _et).  A SpecSrc describes the input grids (run r of a batch at r *_rs): fixed-point accumulators acc[q], converted as convert_multi does
 // (out[q] receives the FP32 grid, acc is cleared, the baseline is taken off
 // the transform's input only), or FP32 grids in.
 struct SpecSrc {

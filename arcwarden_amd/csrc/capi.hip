@@ -237,7 +237,7 @@ struct aw_sim {
         acc8.resize(R * 8 * nc);
         acc3.resize(R * 3 * nc);
         src.resize(R * 11 * nc);
-        if (!ctx->own_fft) fftin.resize(R * 11 * nc);  // [run][4] R2C inputs, then [run][7]
+        if (!ctx->own_em) fftin.resize(R * 11 * nc);  // [run][4] R2C inputs, then [run][7]
         elb.resize(R * 5 * nc);
         et.resize(R * 3 * nc);
         e3.resize(R * 3 * nc);
@@ -245,7 +245,7 @@ struct aw_sim {
         inv.resize(R * 11);
         cdcu.resize(R);
         fmax_part.resize(R * (size_t)std::max(dcu_part_capacity(),
-                                              ctx->own_fft ? 2 * spec_blocks(*ctx, 5) : 0));
+                                              ctx->own_em ? 2 * spec_blocks(*ctx, 5) : 0));
         // static per-quantity fixed-point scales: the per-contribution bound maps
         // to 2^48, leaving 2^14 bound-sized contributions of headroom per cell
         double wmax = w_uniform;
@@ -308,7 +308,7 @@ struct aw_sim {
             j_staggered = false;
         }
         moments_ready = false;
-        if (ctx->own_fft) {
+        if (ctx->own_em) {
             solve_fields_own(t);
             return;
         }

@@ -282,7 +282,7 @@ struct aw_ensemble {
             const int64_t nc = ncell(c);
             unsigned long long* counter = g == 0 ? strays.get() : nullptr;
             const int ncounter = g == 0 ? (int)runs.size() : 0;
-            if (!c.own_fft) {
+            if (!c.own_es) {
                 fix_to_float_add(acc.get() + gr.cbase, rho.get() + gr.cbase, nc * gr.count,
                                  fix_log2, true, sg, true, counter, rin.get() + gr.cbase, ncounter,
                                  rbase.get() + gr.cbase);

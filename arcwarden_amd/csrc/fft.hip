@@ -16,7 +16,8 @@
 // above 17).  A step with two markers a cell, electrostatic / Darwin, us:
 // 64x64 24 / 60 (rocFFT 25 / 71), 60x48 25 / 64 (36 / 118), 125x100 27 / 68
 // (47 / 116), 190x250 33 / 94 (54 / 142), 256x256 30 / 99 (32 / 106), 300x300
-// 32 / 104 (49 / 149), 600x400 43 / 174 (52 / 188), 61x61 41 / 146 (82 / 191).
+// 32 / 104 (49 / 149), 600x384 43 / 174 (54 / 194), 61x61 40 / 112 (82 / 200).
+// Where rocFFT is ahead the solves stay with it: ahead(), below.
 #include "fft_device.hpp"
 
 #include <algorithm>
@@ -449,9 +450,9 @@ rows_inverse_kernel(const float2* __restrict__ ks, FftLine fx, int ny, double sc
 
 // Factors n for the line transforms; false past the largest prime whose direct
 // sum was measured ahead of rocFFT's convolution (97x80, above it, takes 47 us
-// a step there).
+// a step there).  direct: the terms of the direct sums are added to it.
 constexpr int kMaxPrime = 61;
-bool make_line(int n, FftLine& l) {
+bool make_line(int n, FftLine& l, int& direct) {
     int f[64], nf = 0, m = n;
     for (; m % 4 == 0; m /= 4) f[nf++] = 4;
     for (; m % 2 == 0; m /= 2) f[nf++] = 2;
@@ -472,6 +473,7 @@ bool make_line(int n, FftLine& l) {
         l.radices |= (unsigned long long)r << (8 * i);
         // a butterfly takes powers of one twiddle, a direct sum any of them
         const bool fly = r <= 5;
+        if (!fly) direct += r;
         l.ntw = std::max(l.ntw, ns == 1 && fly ? 0 : fly ? n / r : n);
         ns *= r;
     }
@@ -504,7 +506,7 @@ int columns_log(const aw_ctx& c, int nmax, int runs) {
 template <class Op>
 void solve(aw_ctx& c, const SpecSrc& in, const SpecDst& out, const Op& op, int runs,
            unsigned int* smax, hipStream_t s) {
-    AW_REQUIRE(c.own_fft, "the grid's solves go through rocFFT");
+    AW_REQUIRE(Op::kIn > 2 ? c.own_em : c.own_es, "the grid's solves go through rocFFT");
     constexpr int NM = std::max(Op::kIn, Op::kOut);
     const int64_t nk = nkmodes(c);
     const int ny = c.g.ny;
@@ -536,17 +538,53 @@ void solve(aw_ctx& c, const SpecSrc& in, const SpecDst& out, const Op& op, int r
     AW_LAUNCH_CHECK();
 }
 
+// Where the own transforms are ahead of rocFFT, for the electrostatic solve (one
+// grid in, two out) and the Darwin ones (em: up to seven).  They save launches,
+// while rocFFT's passes are cheaper once the launches are full, so it is a
+// matter of size: measured on 300 grids from 24x17 to 3600x600 at two markers a
+// cell, us a step below as own / rocFFT.  A grid's choice does not ask how many
+// runs a batch holds: a run equals the same run stepped alone.
+bool ahead(int nx, int ny, int direct, bool em) {
+    auto pow2 = [](int n) { return (n & (n - 1)) == 0; };
+    const int64_t cells = (int64_t)nx * ny;
+    // rocFFT takes an odd real line as a complex one and falls behind (Darwin
+    // 1001x1: 69 / 123, 61x61: 112 / 200, 625x625: 246 / 320) but for a long line
+    // of direct sums (3599x1, 120 terms: 236 / 212; 3111x78, 78 terms in a row:
+    // 306 / 431)
+    if (nx % 2) return (int64_t)nx * direct <= 400000 && cells <= (int64_t)1 << 19;
+    // work that no launch hides; 24 terms of direct sums weigh as much as all
+    // other passes (610x610, 122 terms: Darwin 531 / 414).  Electrostatic
+    // 2500x384: 81 / 87, 2500x600: 119 / 111; Darwin 960x360: 212 / 244,
+    // 600x600: 249 / 240, 1200x360: 278 / 264, 3000x600: 935 / 703
+    if (cells * (24 + direct) > 24 * (em ? (int64_t)350000 : (int64_t)1 << 20)) return false;
+    // rocFFT's best sides.  Electrostatic 256x256: 29.7 / 31.9, 512x64: 28.5 /
+    // 29.1, 512x128: 31.6 / 28.4; Darwin 1024x64: 95 / 100, 128x512: 108 / 102,
+    // 2048x1: 67 / 63
+    if (pow2(nx) && pow2(ny)) {
+        const int side = std::max(nx, ny);
+        if (em) return nx <= 1024 && ny <= 256;
+        return side <= 256 || (side <= 512 && cells <= 1 << 15);
+    }
+    // long rows, and too few of them for the chip.  Darwin 1300x1: 69 / 76,
+    // 1400x1: 68 / 64, 3600x1: 84 / 76, 3000x17: 113 / 99, 3000x60: 137 / 143
+    if (em) return nx <= 1300 || ny > 60;
+    // long rows and columns that rocFFT is good at.  Electrostatic 625x1: 22 / 37,
+    // 1250x128: 36.6 / 32.6, 1250x1: 24.2 / 22.9, 3000x100: 50 / 48; 1000x120:
+    // 34 / 45, 3000x250: 67 / 79
+    if (direct == 0 && nx > 512 && ny > 1 && pow2(ny)) return false;
+    return nx <= 1200 || ny > 100;
+}
+
 }  // namespace
 
 // The grids whose solves run here: sides made of the transforms' factors, lines
-// (at most a column of E_T's seven grids) that fit LDS.
+// (at most a column of E_T's seven grids) that fit LDS, and where that is ahead.
 void init_own_fft(aw_ctx& c) {
-    c.own_fft = false;
-    if (!make_line(c.g.nx, c.fx) || !make_line(c.g.ny, c.fy)) return;
-    // rocFFT's best sides at a size that fills the chip: 40 / 169 us a step at
-    // 512x512 against 43 / 196 here, while at 256x256 it is behind
-    auto pow2 = [](int n) { return (n & (n - 1)) == 0; };
-    if (pow2(c.g.nx) && pow2(c.g.ny) && ncell(c) >= (int64_t)1 << 18) return;
+    c.own_es = c.own_em = false;
+    int direct = 0;
+    if (!make_line(c.g.nx, c.fx, direct) || !make_line(c.g.ny, c.fy, direct)) return;
+    const bool es = ahead(c.g.nx, c.g.ny, direct, false), em = ahead(c.g.nx, c.g.ny, direct, true);
+    if (!es && !em) return;
     if (rows_lds(c) + kRowsStaticLds > c.lds_per_block ||
         columns_lds(c, 7, 1) > c.lds_per_block)
         return;
@@ -566,7 +604,8 @@ void init_own_fft(aw_ctx& c) {
     AW_HIP(hipMemcpy(c.fft_tw.get(), tw.data(), tw.size() * sizeof(double2), hipMemcpyHostToDevice));
     c.fx.tw = c.fft_tw.get();
     c.fy.tw = c.fft_tw.get() + c.g.nx;
-    c.own_fft = true;
+    c.own_es = es;
+    c.own_em = em;
 }
 
 // workgroups a run of the rows-inverse launch (the pairs of maxima of kFormEl)

@@ -1,7 +1,7 @@
 // spectral.hip -- rocFFT plans and the pointwise k-space solves, for the grids
-// whose sides the library's own transforms (fft.hip) do not take: a prime
-// factor above 61, lines too long for LDS, or large powers of two.  The entry
-// points below choose.
+// that the library's own transforms (fft.hip) leave: a prime factor above 61,
+// lines too long for LDS, and where rocFFT is ahead.  The entry points below
+// choose.
 //
 // Reference: CufftPlan2D (include/pic/fft.hpp:26-93), SpectralEngine
 // (include/pic/spectral.hpp:106-149), es_poisson_field_kernel
@@ -100,11 +100,11 @@ void init_fft(aw_ctx& c) {
     init_own_fft(c);
     c.r2c = make_plan(c, true, 1, 1.0);  // aw_fft_r2c, aw_fft_c2r
     c.c2r = make_plan(c, false, 1, inv);
-    if (!c.own_fft) {
+    if (!c.own_es) {
         c.c2r2 = make_plan(c, false, 2, inv);
         c.r2c2 = make_plan(c, true, 2, 1.0);
-        c.c2r3 = make_plan(c, false, 3, inv);
     }
+    if (!c.own_em) c.c2r3 = make_plan(c, false, 3, inv);
     size_t work = 0;
     for (rocfft_plan p : {c.r2c, c.c2r, c.c2r2, c.r2c2, c.c2r3}) {
         if (!p) continue;
@@ -119,7 +119,7 @@ void init_fft(aw_ctx& c) {
 // Darwin batches: R2C x4 [rho|Jx|Jy|Jz], R2C x7 [dcu(3)|amu(4)], C2R x5
 // [ELx|ELy|Bx|By|Bz] (C2R x3 [ETx|ETy|ETz] is shared with the base set).
 void enable_em_fft(aw_ctx& c) {
-    if (c.own_fft || c.r2c4) return;
+    if (c.own_em || c.r2c4) return;
     const double inv = 1.0 / ((double)c.g.nx * (double)c.g.ny);
     c.r2c4 = make_plan(c, true, 4, 1.0);
     c.r2c7 = make_plan(c, true, 7, 1.0);
@@ -137,7 +137,7 @@ void enable_em_fft(aw_ctx& c) {
 void enable_em_batch_fft(aw_ctx& c, int R) {
     if (c.em_batch == R) return;
     AW_REQUIRE(c.em_batch == 0, "Darwin batch plans already prepared for another size");
-    if (c.own_fft) {
+    if (c.own_em) {
         c.em_batch = R;
         return;
     }
@@ -207,7 +207,7 @@ std::pair<SpecSrc, SpecDst> own_grids(aw_ctx& c, const float* src, int nin, floa
 void convert_solve_es(aw_ctx& c, unsigned long long* acc, float* rho, float* E2, double eps0,
                       unsigned long long* counter, hipStream_t s) {
     const int64_t nc = ncell(c);
-    if (!c.own_fft) {
+    if (!c.own_es) {
         c.rin.reserve((size_t)nc);
         fix_to_float_add(acc, rho, nc, c.fix_log2, true, s, true, counter, c.rin.get(), 1, nullptr,
                          c.rho_base);
@@ -271,7 +271,7 @@ __global__ void es_kspace_batch_kernel(const float2* __restrict__ rk, float2* __
 
 void enable_batch_fft(aw_ctx& c, int batch) {
     if (c.fft_batch == batch) return;
-    if (c.own_fft) {
+    if (c.own_es) {
         c.fft_batch = batch;
         return;
     }
@@ -294,10 +294,10 @@ void enable_batch_fft(aw_ctx& c, int batch) {
 }
 
 // rho_in: B grids [B][ny][nx] (rocFFT may overwrite them); E2B: [B][Ex|Ey].
-// Only where the solves are rocFFT's (not own_fft).
+// Only where the solves are rocFFT's (not own_es).
 void solve_es_batch(aw_ctx& c, int batch, float* rho_in, float* E2B, double eps0,
                     hipStream_t s) {
-    AW_REQUIRE(c.fft_batch == batch && !c.own_fft, "batched plans not prepared for this batch");
+    AW_REQUIRE(c.fft_batch == batch && !c.own_es, "batched plans not prepared for this batch");
     const int64_t nk = nkmodes(c);
     c.ktmp.reserve((size_t)6 * nk * batch);
     float2* rk = reinterpret_cast<float2*>(c.ktmp.get());
@@ -311,7 +311,7 @@ void solve_es_batch(aw_ctx& c, int batch, float* rho_in, float* E2B, double eps0
 }
 
 void solve_es_contig(aw_ctx& c, const float* rho, float* E2, double eps0, hipStream_t s) {
-    if (c.own_fft) {
+    if (c.own_es) {
         own_es(c, rho, E2, E2 + ncell(c), eps0, s);
         return;
     }
@@ -442,7 +442,7 @@ __global__ void darwin_et_kernel(const float2* __restrict__ src, float2* __restr
 void solve_darwin_elb(aw_ctx& c, const float* src4, float* out5, double eps0, double cl,
                       const float B0[3], hipStream_t s, bool stag, int runs) {
     AW_REQUIRE(runs == 1 || runs == c.em_batch, "Darwin batch plans not prepared");
-    if (c.own_fft) {
+    if (c.own_em) {
         const auto [in, out] = own_grids(c, src4, 4, out5, 5);
         spec_solve_elb(c, in, out, eps0, cl, B0, stag, runs, s);
         return;
@@ -464,7 +464,7 @@ void solve_darwin_elb(aw_ctx& c, const float* src4, float* out5, double eps0, do
 void solve_darwin_et(aw_ctx& c, const float* src7, float* out3, double eps0, double cl,
                      double n0, hipStream_t s, int runs) {
     AW_REQUIRE(runs == 1 || runs == c.em_batch, "Darwin batch plans not prepared");
-    if (c.own_fft) {
+    if (c.own_em) {
         const auto [in, out] = own_grids(c, src7, 7, out3, 3);
         spec_solve_et(c, in, out, eps0, cl, n0, runs, s);
         return;
@@ -483,7 +483,7 @@ void solve_darwin_et(aw_ctx& c, const float* src7, float* out3, double eps0, dou
 
 // General form with separate output buffers.
 void solve_es(aw_ctx& c, const float* rho, float* Ex, float* Ey, double eps0, hipStream_t s) {
-    if (c.own_fft) {
+    if (c.own_es) {
         own_es(c, rho, Ex, Ey, eps0, s);
         return;
     }

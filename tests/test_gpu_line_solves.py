@@ -2,8 +2,7 @@
 E of rho, E_L and B of [rho|J], E_T of [dcu|amu] against the same algebra on
 numpy's FP64 transforms, over sides of every factor the transforms have a pass
 for (5, 4, 3, 2, other primes to 61), odd, prime and one-row grids, the
-longest line, and sides that stay with rocFFT (a prime above 61, a line that
-leaves no LDS for what else its kernels hold).
+longest line, and sides of which one kind of solve or both stay with rocFFT.
 
 The library's transforms are FP64 between three FP32 roundings of every value
 (the two half spectra and the result), 2^-24 at most and independent: below
@@ -19,18 +18,17 @@ from arcwarden_amd import _lib as L
 
 pytestmark = pytest.mark.gpu
 
-SIDES = [(64, 64), (128, 96), (250, 190), (33, 17), (61, 59), (7, 121), (243, 125), (16, 1),
-         (4096, 1), (3001, 1), (1000, 1), (2, 2), (3, 5), (1, 24), (512, 96), (40, 600),
-         (67, 40), (40, 134), (512, 512), (3150, 1), (3150, 16)]
-
-
-def _own(n):
-    p, m = 2, n
-    while p * p <= m:
-        while m % p == 0:
-            m //= p
-        p += 1
-    return (m if m > 1 else 1) <= 61 or n == 1
+# on the library's own transforms
+OWN = [(64, 64), (128, 96), (250, 190), (33, 17), (61, 59), (7, 121), (243, 125), (16, 1),
+       (1000, 1), (3125, 1), (2, 2), (3, 5), (1, 24), (512, 96), (40, 600), (625, 625)]
+# the electrostatic solve only, and the Darwin ones only
+OWN_ES = [(64, 512), (2500, 360), (1200, 360), (3000, 110)]
+OWN_EM = [(1024, 64), (512, 128), (1250, 128), (3000, 100)]
+# rocFFT: a prime above 61, a line longer than LDS, one that leaves no LDS for
+# what else its kernels hold (3150: 163,808 of 163,840 bytes), and the sides where
+# rocFFT is ahead
+ROCFFT = [(67, 40), (40, 134), (3001, 1), (4096, 1), (3150, 62), (3150, 110), (512, 512),
+          (2048, 1), (3599, 1)]
 
 
 def _kvec(nx, ny, dx, dy):
@@ -77,7 +75,7 @@ def solver(gpu):
         L.lib().aw_ctx_destroy(h)
 
 
-@pytest.mark.parametrize("nx,ny", SIDES)
+@pytest.mark.parametrize("nx,ny", OWN + OWN_ES + OWN_EM + ROCFFT)
 def test_solves_match_fp64(solver, nx, ny):
     dx, dy, eps0, c, n0 = 0.5, 0.4, 1.3, 7.0, 0.9
     ctx = solver(nx, ny, dx, dy)
@@ -97,18 +95,15 @@ def test_solves_match_fp64(solver, nx, ny):
     torch.cuda.synchronize()
     assert np.array_equal(d.cpu().numpy(), src)  # the inputs stay as they are
 
-    # a line of 3150 takes 163,808 bytes of a workgroup's 163,840 and the row
-    # kernels up to 192 of their own: rocFFT
-    own = (_own(nx) and _own(ny) and max(nx, ny) <= 4000 and nx * ny < 1 << 18
-           and nx != 3150)
-    tol = 3.6e-7 if own else 5e-6
+    tol_es = 3.6e-7 if (nx, ny) in OWN + OWN_ES else 5e-6
+    tol = 3.6e-7 if (nx, ny) in OWN + OWN_EM else 5e-6
     kx, ky, nyq, i, j = _kvec(nx, ny, dx, dy)
     k2 = kx ** 2 + ky ** 2
     on = (k2 > 0) & ~nyq
     safe = np.where(on, k2, 1.0)
     s = np.fft.rfft2(src.astype(np.float64))
     E = [np.where(on, -1j * k * s[0] / (eps0 * safe), 0) for k in (kx, ky)]
-    _check(e.cpu().numpy(), _inverse(E, nx, ny), tol)
+    _check(e.cpu().numpy(), _inverse(E, nx, ny), tol_es)
     for got, stag in ((elb, False), (elbs, True)):
         jx, jy, jz = s[1], s[2], s[3]
         if stag:
