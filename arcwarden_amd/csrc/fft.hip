@@ -71,12 +71,14 @@ int line_ld(int n) { return n + (n >> 3) + 1; }
 constexpr int kMaxWaves = 16;
 constexpr size_t kRowsStaticLds = kMaxWaves * (sizeof(int) + 2 * sizeof(float));
 
-// Which of a thread's two lines hold anything, over the workgroup: bit 0 and 1.
-// A line of zeros comes out as zeros, not as the rounding of its partner.
-// Every thread calls it; a barrier is inside.
-__device__ __forceinline__ int lines_set(bool a, bool b) {
+// What a workgroup's two lines hold: bit 0 and 1 something, bit 2 and 3 a value
+// that is not finite.  A line of zeros comes out as zeros, not as the rounding
+// of its partner.  Every thread calls it; a barrier is inside.
+constexpr int kNotFinite = 4;
+__device__ __forceinline__ int lines_set(bool a, bool b, bool bada = false, bool badb = false) {
     __shared__ int s_set[kMaxWaves];
-    const int m = (__ballot(a) ? 1 : 0) | (__ballot(b) ? 2 : 0);
+    const int m = (__ballot(a) ? 1 : 0) | (__ballot(b) ? 2 : 0) |
+                  (__ballot(bada) ? kNotFinite : 0) | (__ballot(badb) ? 2 * kNotFinite : 0);
     if ((threadIdx.x & 63) == 0) s_set[threadIdx.x >> 6] = m;
     __syncthreads();
     int all = 0;
@@ -127,7 +129,7 @@ rows_forward_kernel(SpecSrc a, FftLine fx, int ny, float2* __restrict__ ks) {
     const Pair p = pair_of(blockIdx.x, NQ, ny);
     const Cell ca(a, nc, r, p.q0), cb(a, nc, r, p.q1);
     const int64_t ra = (int64_t)p.j0 * nx, rb = p.two ? (int64_t)p.j1 * nx : ra;
-    bool seta = false, setb = false;
+    bool seta = false, setb = false, bada = false, badb = false;
     const double2 w0 = fx.tw[min(tid, nx - 1)];
     if constexpr (ACC) {
         const double sa = ca.inv(), sb = cb.inv();
@@ -169,26 +171,31 @@ rows_forward_kernel(SpecSrc a, FftLine fx, int ny, float2* __restrict__ ks) {
             for (int u = 0; u < kAhead; ++u) {
                 const int x = x0 + u * nt + tid;
                 if (x >= nx) continue;
-                const double2 v = make_double2(va[u], p.two ? vb[u] : 0.f);
+                double2 v = make_double2(va[u], p.two ? vb[u] : 0.f);
                 seta = seta || v.x != 0.0;
                 setb = setb || v.y != 0.0;
+                // infinities and NaN stay out of the line they would share
+                if (!isfinite(v.x)) bada = true, v.x = 0.0;
+                if (!isfinite(v.y)) badb = true, v.y = 0.0;
                 s_l[pad(x)] = v;
             }
         }
     }
     if (tid < fx.ntw) s_tw[tid] = w0;
     for (int i = tid + nt; i < fx.ntw; i += nt) s_tw[i] = fx.tw[i];
-    const int set = lines_set(seta, setb);
+    const int set = lines_set(seta, setb, bada, badb);
     const double2* z = lines<-1>(s_l, s_l + ld, fx, s_tw, 1, ld);
     float2* k0 = ks + (((int64_t)r * NQ + p.q0) * ny + p.j0) * nkx;
     float2* k1 = ks + (((int64_t)r * NQ + p.q1) * ny + p.j1) * nkx;
+    // a line that is not finite has no finite mode; its partner is its own
+    const float2 zero = make_float2(0.f, 0.f), none = make_float2(NAN, NAN);
     for (int k = tid; k < nkx; k += nt) {
         const double2 u = z[pad(k)], w = z[pad(k ? nx - k : 0)];
         // the transforms of a and b out of that of a + i b
         const float2 A = make_float2((float)(0.5 * (u.x + w.x)), (float)(0.5 * (u.y - w.y)));
         const float2 B = make_float2((float)(0.5 * (u.y + w.y)), (float)(0.5 * (w.x - u.x)));
-        k0[k] = set & 1 ? A : make_float2(0.f, 0.f);
-        if (p.two) k1[k] = set & 2 ? B : make_float2(0.f, 0.f);
+        k0[k] = set & kNotFinite ? none : set & 1 ? A : zero;
+        if (p.two) k1[k] = set & 2 * kNotFinite ? none : set & 2 ? B : zero;
     }
 }
 

@@ -122,6 +122,37 @@ def test_solves_match_fp64(solver, nx, ny):
     _check(et.cpu().numpy(), _inverse([-G * v for v in J], nx, ny), tol)
 
 
+@pytest.mark.parametrize("nx,ny", [(96, 50), (33, 17), (67, 40)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_values_that_are_not_finite_stay_in_their_fields(solver, nx, ny, bad):
+    """Two grids share a line of the transforms, but only the fields that depend
+    on a grid lose their values with it (the last side is rocFFT's)."""
+    ctx = solver(nx, ny, 0.5, 0.4)
+    src = np.random.default_rng(nx).normal(size=(11, ny, nx)).astype(np.float32)
+    b0 = (C.c_float * 3)(0.3, -0.2, 0.1)
+
+    def fields(at=None):
+        d = torch.from_numpy(src).cuda()
+        if at is not None:
+            d[at, ny // 2, nx // 3] = bad
+        elb, et = torch.zeros(5, ny, nx, device="cuda"), torch.zeros(3, ny, nx, device="cuda")
+        L.call("aw_solve_darwin_el_b", ctx, d.data_ptr(), elb.data_ptr(), 1.0, 7.0, b0, None)
+        L.call("aw_solve_darwin_et", ctx, d[4].data_ptr(), et.data_ptr(), 1.0, 7.0, 0.9, None)
+        torch.cuda.synchronize()
+        return torch.cat([elb, et]).cpu().numpy()
+
+    clean = fields()
+    # grid -> the fields made of it: ELx ELy Bx By Bz ETx ETy ETz
+    for at, of in {1: (4,), 2: (4,), 3: (2, 3), 6: (7,), 7: (5, 6), 10: (7,)}.items():
+        got = fields(at)
+        for q in range(8):
+            if q in of:
+                assert not np.isfinite(got[q]).any(), (at, q)
+            else:
+                err = np.linalg.norm(got[q] - clean[q]) / np.linalg.norm(clean[q])
+                assert err < 1e-6, (at, q, err)
+
+
 def test_darwin_solves_captured_after_the_first(solver):
     """Once one Darwin solve has run, a graph captures both (nothing is left to
     allocate); every replay equals the eager result of the same inputs."""
