@@ -91,6 +91,23 @@ def test_esirkepov_continuity_reference_setup(gpu, oracle):
     assert res_gpu < 5e-5  # the reference's own gate, with FP32 rho storage
 
 
+# tiles whose current leaves LDS for five slots of the move queue a wavefront,
+# for one, and for none (then every move is deposited on the spot)
+@pytest.mark.parametrize("tx,ty", [(78, 79), (58, 106), (61, 101)])
+def test_esirkepov_large_tiles(gpu, tx, ty):
+    """The binned deposit on tiles that fill LDS equals the global atomics bit
+    for bit, most moves leaving their cell."""
+    nx, ny, dx, dy = 2 * tx - 3, 2 * ty + 5, 0.7, 1.3
+    dt, qm = 0.9 * dx, -1.0
+    rng = np.random.default_rng(tx)
+    mv = _moves(rng, nx, ny, 40_000, dx, dy, dt)
+    with Ctx(L.grid(nx, ny, nx * dx, ny * dy), tx, ty) as ctx:
+        a, b = (_gpu_j(ctx, nx, ny, *mv, 0.0, qm, dt, pol)
+                for pol in (L.AW_DEPOSIT_GLOBAL, L.AW_DEPOSIT_BINNED))
+    for q in range(3):
+        assert np.abs(a[q]).max() > 0 and np.array_equal(a[q], b[q]), q
+
+
 @pytest.mark.parametrize("nx,ny,tile,n,by_x", [(128, 96, 16, 1_000_000, False),
                                                (40, 24, 8, 300_000, False),
                                                (16, 4, 16, 5_000, False),

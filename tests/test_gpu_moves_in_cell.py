@@ -1,10 +1,13 @@
-"""GPU test of the split current deposit: moves that stay in their cell are
+"""GPU tests of the split current deposit: moves that stay in their cell are
 deposited on the spot with the 8 contributions that are not zero, the others
-are set aside and take the general stencil (esk_device.hpp).  The tile-ordered
-Yee step does so; the unsorted one on a grid whose current fits LDS deposits
-every move with the general stencil.  Fields and particles must be the same
-bits at every share of moves that leave their cell, on one-row, one-column and
-ragged grids, with uniform and per-particle weights."""
+are set aside and take the general stencil (esk_device.hpp).
+
+The tile-ordered Yee step does so.  The unsorted one deposits every move with
+the general stencil on a grid of several rows whose current fits LDS: fields
+and particles must be the same bits at every share of moves that leave their
+cell, on one-column and ragged grids, with uniform and per-particle weights.
+On one row the unsorted step splits the moves too (its own kernel): there both
+are compared with the FP64 current of the same moves as well."""
 import numpy as np
 import pytest
 
@@ -50,6 +53,40 @@ def test_split_deposit_matches_the_general_stencil(gpu, nx, ny, per_w, step):
     assert step == 0.0 or np.abs(M0[-3 * nx * ny:]).max() > 0
     assert np.array_equal(M0, M1)
     assert np.array_equal(P0, P1)
+
+
+@pytest.mark.parametrize("tile_sort", [0, 1])
+@pytest.mark.parametrize("step", [0.02, 0.5, 0.98])
+@pytest.mark.parametrize("nx,per_w", [(300, False), (17, True), (2, False)])
+def test_one_row_split_deposit_matches_fp64(gpu, oracle, nx, per_w, step, tile_sort):
+    """One step without fields: the particles keep their velocities, and J is the
+    FP64 Esirkepov current of their moves within the FP32 result's rounding."""
+    dx, dt, n = 0.5, 0.05, max(4000, 40 * nx) + 11
+    rp = L.run_params(dt=dt, qm=-1.0, eps0=1.0, c=6.0)
+    rp.tile_sort = tile_sort
+    rng = np.random.default_rng(nx)
+    st = {"x": rng.uniform(0, nx, n).astype(np.float32),
+          "y": rng.uniform(0, 1, n).astype(np.float32)}
+    st["x"][st["x"] >= nx], st["y"][st["y"] >= 1] = 0, 0
+    st["x"][:64] = np.floor(st["x"][:64])
+    for k in ("ux", "uy", "uz"):
+        st[k] = (rng.uniform(-1, 1, n) * step * dx / dt).astype(np.float32)
+    st["uy"] *= 0.5  # half a cell: further, the periodic image on one row is ambiguous
+    w = rng.uniform(0.5, 1.5, n).astype(np.float32) * (dx * dx / 16) if per_w else None
+    wu = 0.0 if per_w else dx * dx / 16
+    sim = MaxwellSimulation(L.grid(nx, 1, nx * dx, dx), rp)
+    sim.set_particles(st, w=w, **({} if per_w else {"w_uniform": wu}))
+    sim.step()
+    sim.synchronize()
+    J = sim.mesh_flat()[6 * nx:].reshape(3, 1, nx)
+    sim.close()
+    og = oracle.grid(nx, 1, dx, dx)
+    x1 = st["x"] + (st["ux"].astype(np.float64) * dt / dx).astype(np.float32)
+    y1 = st["y"] + (st["uy"].astype(np.float64) * dt / dx).astype(np.float32)
+    ref = oracle.esirkepov_f64(og, st["x"], st["y"], x1, y1, st["uz"], -1.0, dt, w=w,
+                               w_uniform=wu)
+    for q in range(3):
+        assert np.linalg.norm(J[q] - ref[q]) < 1e-6 * np.linalg.norm(ref[q]), q
 
 
 @pytest.mark.parametrize("step", [0.01, 0.4, 0.9])

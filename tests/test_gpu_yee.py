@@ -5,8 +5,8 @@
   the FP64 Esirkepov restatement, across B0 orientations, the relativistic
   push, delta-f weights (three precisions), the mirror background on a
   one-row grid, reflecting walls and the pump (one-row grids too, whose push
-  and current are one kernel), and the current smoothing in
-  LDS and in global passes;
+  and current are one kernel), and the current smoothing in one tiled launch
+  and with passes left over;
 - the tile_sort path (particles kept in tile order, the current deposited
   from the tile slices of the last sort) bit for bit against the unsorted
   run, full-f and delta-f;
@@ -62,12 +62,17 @@ CASES = {
                                              b0_xc=16.0)),
     "walls_smoothing": (48, 8, 0.5, 0.5, dict(B0=(0.2, 0.0, 0.3), bnd_x=2, bnd_nd=6,
                                               bnd_numax=0.5, jfilter=2)),
-    # grids above the in-LDS smoothing size: the multi-launch passes
+    # the current's smoothing: up to four passes in the tiled launch, the rest
+    # in LDS on a small grid and one launch a pass on a large one
     "smoothing_3_passes_large": (128, 80, 0.5, 0.5, dict(B0=(0.0, 0.3, 0.2), jfilter=3)),
     "smoothing_1_pass_large": (128, 80, 0.5, 0.5, dict(B0=(0.0, 0.3, 0.2), jfilter=1)),
     "pump": (48, 12, 0.5, 0.5, dict(B0=(0.4, 0.0, 0.2), pump=1, pump_ex=1e-3, pump_ey=2e-3,
                                     pump_ez=-2e-3, pump_k0=TWO_PI * 3 / 24.0, pump_w0=0.15,
                                     pump_trmp=0.5, pump_toff=100.0)),
+    "smoothing_4_passes_ragged": (50, 37, 0.5, 0.5, dict(B0=(0.0, 0.3, 0.2), jfilter=4)),
+    "smoothing_5_passes_ragged": (50, 37, 0.5, 0.5, dict(B0=(0.0, 0.3, 0.2), jfilter=5)),
+    "smoothing_6_passes_large": (133, 77, 0.5, 0.5, dict(B0=(0.0, 0.3, 0.2), jfilter=6)),
+    "smoothing_6_passes_one_row": (300, 1, 0.5, 0.5, dict(B0=(0.3, 0.0, 0.0), jfilter=6)),
     # one row at 16 particles a cell or more: the push and the current in one kernel
     "relativistic_one_row": (300, 1, 0.5, 0.5, dict(B0=(0.2, 0.0, 0.4), rel=1)),
     "pump_one_row": (257, 1, 0.5, 0.5, dict(B0=(0.4, 0.0, 0.2), pump=1, pump_ex=1e-3,
