@@ -275,8 +275,9 @@ bool tile_sort_onepass(aw_ctx& c, const aw_particles& src, const aw_particles& d
 void bin_tiles(aw_ctx& c, const aw_particles& p, int32_t* perm, int32_t* off, hipStream_t s);
 
 // p copied in stable tile order into the context's scratch (x, y and w only, or
-// all of it), the offsets in c.sort.bin_off.  False, and nothing done, where
-// the one-pass sort does not apply or the copy has no room.
+// all of it), the offsets in c.sort.bin_off.  False, and nothing sorted, where
+// the one-pass sort does not apply or the copy has no room; the scratch is held
+// as long as the context.
 bool tile_sorted_copy(aw_ctx& c, const aw_particles& p, bool positions_only, aw_particles& out,
                       hipStream_t s);
 
@@ -338,9 +339,11 @@ PumpArgs pump_args(const aw_grid& g, const aw_run_params& rp, double t);
 
 // Solves on the library's own transforms (fft.hip), which fuse the fixed-point
 // conversion before them and the field combination after them; only where
-// own_es (spec_solve_es, _adj) or own_em (_elb, _et).  A SpecSrc describes the input grids (run r of a batch at r *_rs): fixed-point accumulators acc[q], converted as convert_multi does
-// (out[q] receives the FP32 grid, acc is cleared, the baseline is taken off
-// the transform's input only), or FP32 grids in.
+// own_es (spec_solve_es, _adj) or own_em (_elb, _et).  A SpecSrc describes the
+// input grids (run r of a batch at r *_rs): fixed-point accumulators acc[q],
+// converted as convert_multi does (out[q] receives the FP32 grid, acc is
+// cleared, the baseline is taken off the transform's input only), or FP32 grids
+// in.
 struct SpecSrc {
     // grids q < split from acc + q nc, the others from acc2 + (q - split) nc
     unsigned long long *acc = nullptr, *acc2 = nullptr;

@@ -924,8 +924,8 @@ int dcu_part_capacity() { return 2 * 256; }
 // aw_deposit_rho_j_amu, aw_deposit_dcu and aw_push_boris_em take particles in
 // any order.  The deposits sort a copy of them by tile (or, without room for
 // it, bin them into the context's permutation and read them through it); their
-// fixed-point scales come from the measured max |w| and max |u|.  The push gathers from
-// the packed grid.
+// fixed-point scales come from the measured max |w| and max |u|.  The push
+// gathers from the packed grid.
 
 // q = p in tile order and no permutation, or p itself and the bins of its tiles
 static const int32_t* bin_particles(aw_ctx& c, const aw_particles& p, aw_particles& q,

@@ -3,7 +3,7 @@
 // Stockham passes (no bit reversal): radix 5, 4, 3 and 2 butterflies in
 // registers and a direct sum for any other prime, so that every length works.
 // A workgroup holds a line or a few, so a pass lasts as long as one lane's
-// butterfly: 1000 cycles at radix 4 and 2200 at radix 8, whose 273 instructions
+// butterfly: 1500 cycles at radix 4 and 2200 at radix 8, whose 273 instructions
 // leave 7 of 8 lanes idle on a line of 64.  Lines sit in LDS `ld` elements
 // apart with one element of padding in nine, which keeps the strided stores of
 // a first pass off each other's banks.  On this card an FP64 multiply-add costs

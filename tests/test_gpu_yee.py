@@ -455,9 +455,10 @@ def test_tile_sort_matches_unsorted(gpu, deltaf, nx, ny):
     tile-sorted run pushes and deposits in one kernel per tile (the plain
     instance without delta-f, the general one with it; one-row grids sum
     their aliased stencil rows); the unsorted one in a push and a deposit
-    (64 x 48, 512 x 1: the current's whole grid fits LDS), or with the same
-    kernel over tile bins of the unmoved arrays (256 x 160, 10 particles per
-    cell)."""
+    (64 x 48: the current's whole grid fits LDS), in one kernel that keeps the
+    row's current (512 x 1; both split the moves there, and
+    test_gpu_moves_in_cell.py has them against FP64), or with the same kernel
+    over tile bins of the unmoved arrays (256 x 160, 10 particles per cell)."""
     M0, P0 = _tile_sort_run(0, deltaf, nx=nx, ny=ny)
     M1, P1 = _tile_sort_run(5, deltaf, nx=nx, ny=ny)
     nc = nx * ny
